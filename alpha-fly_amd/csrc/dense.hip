@@ -29,6 +29,7 @@ namespace fly {
 
 int64_t io_block(const fly_plan &plan, int64_t batch);
 size_t io_workspace(const fly_plan &plan, int64_t batch);
+int64_t run_ld(const fly_plan &plan, int64_t batch, size_t elem);
 size_t plan_pieces_bytes(const fly_plan &plan, int64_t batch);
 template <typename S, typename U>
 const S *run_cone_steps(const fly_plan &plan, const U *u, int64_t ldu, int64_t batch, bool u_padded, void *ws,
@@ -680,7 +681,7 @@ void model_forward_blocks(const fly_plan &plan, const fly_dense &d, const void *
     const void *xb = static_cast<const char *>(x) + (size_t)c0 * ldx * xelem;
     float *lb = logits + c0 * d.n_moves, *wb = wdl + c0 * 3;
     const int64_t ldu = state_ld(nb, sizeof(float));
-    const int64_t lds = state_ld(nb, es);
+    const int64_t lds = run_ld(plan, nb, es);
     // The encoder output stays float32 in both modes: only the deviation state is carried in float16.
     run_encoder(d, xb, x_f16, ldx, nb, input_gain, u, nullptr, ldu, scratch_ops, st);
     if (plan.mode == FLY_MODE_DEVIATION_F16) {

@@ -70,4 +70,30 @@ __device__ __forceinline__ float group_reduce_scatter8(const float (&d)[8], int 
   return (h1 ? f[1] : f[0]) + lane_xor<1>(h1 ? f[0] : f[1]);
 }
 
+// v from the lane (l ^ X), X = 1, 2, 4, 8 or 16: DPP inside 16-lane rows where it has the permutation, else ds_swizzle.
+template <int X>
+__device__ __forceinline__ float lane_xor_dpp(float v) {
+  constexpr int ctrl = X == 1 ? 0xB1 /* quad_perm 1,0,3,2 */ : X == 2 ? 0x4E /* quad_perm 2,3,0,1 */ : 0x128 /* row_ror:8 */;
+  if constexpr (X == 1 || X == 2 || X == 8)
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xF, 0xF, false));
+  else
+    return lane_xor<X>(v);
+}
+
+// One halving exchange of a reduce-scatter between lanes X apart: the lane whose bit X is clear returns the pair's sum
+// of lo, the other one the pair's sum of hi.
+template <int X>
+__device__ __forceinline__ float halve_exchange(float lo, float hi, int lane) {
+  if constexpr (X == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(lo), __float_as_int(hi), false, false);
+    return __int_as_float(r[0]) + __int_as_float(r[1]);
+  } else if constexpr (X == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_int(lo), __float_as_int(hi), false, false);
+    return __int_as_float(r[0]) + __int_as_float(r[1]);
+  } else {
+    const bool up = lane & X;
+    return (up ? hi : lo) + lane_xor_dpp<X>(up ? lo : hi);
+  }
+}
+
 }  // namespace fly

@@ -73,11 +73,80 @@ void launch_v(const StepArgs<S, U> &a, int groups, int unroll, bool rows_mode, i
     hipLaunchKernelGGL((k_state_step<S, U, V, 8, kTL>), grid, block, lds, st, a);
 }
 
+// Whether steps of a plan created under `tune` may run narrow: not where a key asks for another kernel's shape.
+bool narrow_on(const Tuning &tune) {
+  return tune.narrow >= 0 && tune.swept <= 0 && tune.vec == 0 && tune.groups == 0 && tune.rows_mode == 0;
+}
+
+// The narrow kernel for batches of up to 32 bytes a row, where the rows' 16-byte (2- or 4-byte) pieces can be read.
+template <typename S, typename U, int V, int L>
+void launch_narrow(StepArgs<S, U> &a, const Tuning &tune, hipStream_t st) {
+  a.u_vec = 0;
+  a.nt_store = tune.nt_store;
+  a.nt_load = tune.nt_load;
+  LaunchTimer timer(FLY_K_STATE_STEP, st);
+  hipLaunchKernelGGL((k_state_step_narrow<S, U, V, L, sizeof(S) == 4>), dim3(blocks_for(blocks_for(a.nrows, 4 / L), 4)),
+                     dim3(256), 0, st, a);
+  check_launch("narrow state step");
+}
+
+// Workgroups of a staged step: one per CU, at least one row block on each XCD; and the rows it takes at most (a unit of
+// 16 lanes keeps a 64-bit mask of its quads of rows).
+unsigned stage_grid(const StageTables &t) {
+  return (unsigned)std::max<int64_t>(round_up(cu_count(), 8), 8 * t.bands);
+}
+int64_t stage_rows(const StageTables &t) { return (int64_t)4 * 64 * 64 * 8 * (stage_grid(t) / 8 / t.bands); }
+
+template <typename S, typename U, int NC>
+void launch_staged(StepArgs<S, U> &a, const StageTables &t, const Tuning &tune, int64_t prev_rows, hipStream_t st) {
+  a.u_vec = 0;
+  a.nt_store = tune.nt_store;
+  a.nt_load = tune.nt_load;
+  LaunchTimer timer(FLY_K_STATE_STEP, st);
+  hipLaunchKernelGGL((k_stage_sums<S, NC>), dim3(stage_grid(t)), dim3(1024), 0, st, t.start.p, a.colval, a.xprev,
+                     (int32_t)prev_rows, a.nrows, t.bands, t.band_rows, a.partials);
+  hipLaunchKernelGGL((k_stage_finish<S, U, NC, sizeof(S) == 4>), dim3(blocks_for((int64_t)a.nrows * NC, 256)), dim3(256),
+                     0, st, a, t.bands);
+  check_launch("staged state step");
+}
+
+// Batches of up to 32 bytes a row: the narrow kernel, and the staged sums for long-row steps of up to 4 bytes a row.
+// Why the lines lie there (full-size network, us per forward, before and after): 1 position 397 -> 190 staged, 2
+// positions 397 -> 195 staged, 3 to 8 397 -> 275 narrow, 9 to 16 397 -> 335 narrow.  At 17 to 32 positions (64 bytes a
+// row) the narrow kernel took 426 against 399, since its 10.7 MB of source rows overflow an XCD's L2; there the wide
+// kernels run on 64-byte state rows (387: half the lines of a band).  Staged rows of 8 bytes would serve 4 positions, but
+// a board would then sum in another order at 4 positions than at 5.
+template <typename S, typename U>
+bool narrow_step(StepArgs<S, U> &a, const Tuning &tune, const SweepTables *sweep, hipStream_t st) {
+  constexpr int E = (int)sizeof(S), V = 16 / E;
+  const int64_t bytes = narrow_ld(a.batch, E) * E;
+  if (!narrow_on(tune) || bytes == 0 || bytes > 32) return false;
+  const int64_t piece = std::min<int64_t>(bytes, 16) / E;
+  if (a.xprev && (a.ldx % piece || !aligned(a.xprev, 16) || !a.xbytes || (a.out_exact && a.batch % piece))) return false;
+  if (bytes <= 4) {
+    const StageTables *t = sweep ? &sweep->stage[bytes == 4] : nullptr;
+    const bool staged = t && t->bands && a.nrows <= stage_rows(*t) && a.partials && a.xprev && a.rowptr && a.ldx == piece && a.batch == piece;
+    if (staged) {
+      const int64_t prev_rows = a.xbytes / bytes;
+      if (E == 4 || piece == 1) launch_staged<S, U, 1>(a, *t, tune, prev_rows, st);
+      else if constexpr (E == 2) launch_staged<S, U, 2>(a, *t, tune, prev_rows, st);
+      return true;
+    }
+    if (E == 4 || piece == 1) launch_narrow<S, U, 1, 1>(a, tune, st);
+    else if constexpr (E == 2) launch_narrow<S, U, 2, 1>(a, tune, st);
+    return true;
+  }
+  if (bytes == 16) launch_narrow<S, U, V, 1>(a, tune, st);
+  else launch_narrow<S, U, V, 2>(a, tune, st);
+  return true;
+}
+
 // One state step.  `sweep`: the step matrix's banded-sweep tables (null: the step does not sweep); a.pieces must then
 // hold sweep_pieces_bytes(sweep, batch) bytes.
 template <typename S, typename U>
 void state_step(StepArgs<S, U> a, double avg_nnz, const Tuning &tune, const SweepTables *sweep, hipStream_t st) {
   if (a.nrows == 0 || a.batch == 0) return;
+  if (narrow_step(a, tune, sweep, st)) return;
   Tuning tu = tune;
   if (sweep && tune.swept > 0) tu.rows_mode = -1;   // a forced sweep takes steps of short rows too
   const StepShape sh = shape_step(a, avg_nnz, tu);
@@ -244,6 +313,12 @@ size_t plan_pieces_bytes(const fly_plan &plan, int64_t batch) {
   return plan.max_pieces ? align256((size_t)plan.max_pieces * (size_t)round_up(batch, 64) * sizeof(float)) : 0;
 }
 
+// Row stride of the plan's state buffers at `batch` columns: the batch's own bytes for narrow batches, else state_ld.
+int64_t run_ld(const fly_plan &plan, int64_t batch, size_t elem) {
+  const int64_t ld = narrow_on(plan.tune) ? narrow_ld(batch, elem) : 0;
+  return ld ? ld : state_ld(batch, elem);
+}
+
 size_t io_states_bytes(const fly_plan &plan, int64_t blk) {
   const size_t es = state_bytes(plan);
   return align256(2 * (size_t)plan.max_rows * (size_t)state_ld(blk, es) * es + 256);
@@ -254,15 +329,29 @@ size_t io_workspace(const fly_plan &plan, int64_t batch) {
   return io_states_bytes(plan, blk) + plan_pieces_bytes(plan, blk);
 }
 
+// The two state buffers (rows, ld) at ws, each on a 256-byte boundary, and the scratch of the staged steps' band sums
+// after them for rows of up to 4 bytes (null otherwise).  All of it lies inside the space of two state_ld buffers:
+// those hold at least 128 bytes a row, of which two narrow rows and kStageBands sums of each of their columns take
+// at most 72.
+template <typename S>
+float *place_states(void *ws, int64_t rows, int64_t ld, S *(&buf)[2]) {
+  const size_t bytes = align256((size_t)rows * (size_t)ld * sizeof(S));
+  const bool narrow = ld * (int64_t)sizeof(S) <= 4;
+  buf[0] = static_cast<S *>(ws);
+  buf[1] = narrow ? reinterpret_cast<S *>(static_cast<char *>(ws) + bytes) : buf[0] + (size_t)rows * (size_t)ld;
+  return narrow ? reinterpret_cast<float *>(static_cast<char *>(ws) + 2 * bytes) : nullptr;
+}
+
 // Runs steps 1..T of a light-cone plan.  Returns the final state (null if R_T is empty) in one of the two
-// workspace buffers, whose row stride is state_ld(batch, sizeof(S)).  u_padded: the drive u is the library's own
+// workspace buffers, whose row stride is run_ld(plan, batch, sizeof(S)).  u_padded: the drive u is the library's own
 // workspace, whose rows may be read up to the batch rounded up to 64 columns.  pieces: plan_pieces_bytes(plan,
 // batch) bytes for the sums of split rows.
 template <typename S, typename U>
 const S *run_cone_steps(const fly_plan &plan, const U *u, int64_t ldu, int64_t batch, bool u_padded, void *ws,
                         float *pieces, hipStream_t st) {
-  const int64_t lds = state_ld(batch, sizeof(S));
-  S *buf[2] = {reinterpret_cast<S *>(ws), reinterpret_cast<S *>(ws) + (size_t)plan.max_rows * lds};
+  const int64_t lds = run_ld(plan, batch, sizeof(S));
+  S *buf[2];
+  float *partials = place_states(ws, plan.max_rows, lds, buf);
   const S *prev = nullptr;
   int cur = 0;
   for (int t = 1; t <= plan.steps; ++t) {
@@ -289,6 +378,7 @@ const S *run_cone_steps(const fly_plan &plan, const U *u, int64_t ldu, int64_t b
     a.batch = (int32_t)batch;
     a.xbytes = prev ? buffer_bytes(plan.rows_n[t - 1], lds, sizeof(S)) : 0;
     a.pieces = pieces;
+    a.partials = partials;
     a.sweep_exact = std::isfinite(plan.h_max) ? 0 : 1;   // no upper clamp: a state may overflow to inf
     state_step(a, nr ? (double)plan.nnz[t] / (double)nr : 0.0, plan.tune, plan.sweep[t].get(), st);
     prev = buf[cur];
@@ -301,7 +391,7 @@ template <typename S>
 void write_outputs(const fly_plan &plan, const S *state, int64_t batch, float *out, int64_t ldo, hipStream_t st) {
   if (!plan.n_out || !batch) return;
   LaunchTimer timer(FLY_K_OTHER, st);
-  hipLaunchKernelGGL(k_outputs<S>, rows_grid(plan.n_out, batch), dim3(256), 0, st, state, state_ld(batch, sizeof(S)),
+  hipLaunchKernelGGL(k_outputs<S>, rows_grid(plan.n_out, batch), dim3(256), 0, st, state, run_ld(plan, batch, sizeof(S)),
                      plan.out_src.p, plan.cbase.p,
                      plan.n_out, batch, out, ldo);
   check_launch("outputs");
@@ -441,8 +531,9 @@ void run_literal(const fly_plan *plan, S *u, int64_t ldu, const float *bias, int
       static_cast<char *>(ws) + align256(2 * (size_t)n * (size_t)state_ld(blk, sizeof(S)) * sizeof(S) + 256));
   for (int64_t c0 = 0; c0 < batch; c0 += blk) {
     const int64_t nb = std::min(blk, batch - c0);
-    const int64_t lds = state_ld(nb, sizeof(S));
-    S *buf[2] = {static_cast<S *>(ws), static_cast<S *>(ws) + (size_t)n * lds};
+    const int64_t lds = run_ld(*plan, nb, sizeof(S));
+    S *buf[2];
+    float *partials = place_states(ws, n, lds, buf);
     const S *prev = nullptr;
     int cur = 0;
     for (int t = 1; t <= steps; ++t) {
@@ -462,6 +553,7 @@ void run_literal(const fly_plan *plan, S *u, int64_t ldu, const float *bias, int
       a.batch = (int32_t)nb;
       a.xbytes = prev ? buffer_bytes(n, lds, sizeof(S)) : 0;
       a.pieces = pieces;
+      a.partials = partials;
       a.sweep_exact = std::isfinite(plan->h_max) ? 0 : 1;
       state_step(a, (double)plan->nnz[0] / (double)n, plan->tune, plan->sweep[0].get(), st);
       prev = buf[cur];
@@ -629,6 +721,7 @@ const TuningKey kTuningKeys[] = {
     {"sweep_pipe", &Tuning::sweep_pipe, -kAny, kAny},
     {"step_lds", &Tuning::step_lds, 0, 65536},
     {"nt_load", &Tuning::nt_load, -kAny, kAny},
+    {"narrow", &Tuning::narrow, -1, 0},
     {"sweep_last_sync", &Tuning::sweep_last_sync, 0, 1},
 };
 

@@ -129,6 +129,7 @@ struct StepArgs {
   // row slots of 8 rows: the lead slots (holding a row far longer than the mean) run first, for every chunk
   const int32_t *lead;         // (nlead) the lead slots, rising
   const uint8_t *lead_flag;    // (slots) 1 for a lead slot
+  float *partials;             // scratch of the staged step's band sums (bands, nrows, batch), or null
   int32_t nlead;               // 0: none (and whenever the launch is not row slots of 8 rows, one chunk per tile)
 };
 
@@ -676,6 +677,246 @@ __global__ __launch_bounds__(256) void k_state_step_rows(const StepArgs<S, U> a)
   }
   if (!active) return;
   finish_row<S, U, V, TORCH_LERP>(a, row, col, acc, in);
+}
+
+// ---- narrow batches ------------------------------------------------------------------------------------
+
+// The sum of 16 ways' shares of V columns, way w in the lanes L w .. L w + L - 1 of each 16 L lanes: halving exchanges
+// leave every lane one column's sum (column way / (16 / V)).  The same pairs meet in the same order whatever L and V
+// are.
+template <int STRIDE, int L, int V>
+__device__ __forceinline__ float narrow_sum(const float (&acc)[V], int lane) {
+  if constexpr (V > 1) {
+    float h[V / 2];
+#pragma unroll
+    for (int i = 0; i < V / 2; ++i) h[i] = halve_exchange<STRIDE>(acc[i], acc[i + V / 2], lane);
+    return narrow_sum<STRIDE / 2, L, V / 2>(h, lane);
+  } else {
+    const float v[1] = {acc[0] + lane_xor_dpp<STRIDE>(acc[0])};
+    if constexpr (STRIDE > L) return narrow_sum<STRIDE / 2, L, 1>(v, lane);
+    else return v[0];
+  }
+}
+
+// A step of a batch whose state rows hold L pieces of V columns (one piece of 2, 4 or 16 bytes, or 2 of 16: up to 16
+// half or 8 float columns).  16 ways of L lanes share a row: way w takes the row's non-zeros w, w + 16, ... and each of its lanes one
+// piece of the gathered row, so a wave runs 4 / L rows and a gather moves only the batch's own bytes of a source row.
+// The 16 partial sums meet in a fixed tree that does not depend on L: a board's sums have the same bits whatever the
+// batch around it.  What bounds it: the L1's line fills, one 128-byte line per gather whatever the gather uses of it
+// (10.5M non-zeros over 16-byte rows in 73 us, 143 G lines/s, where the swept kernel took 110 us: it issues 1.27
+// gathers per non-zero and finds two thirds of its 128-byte rows in the L2, this one nearly all of its 16-byte rows).
+template <typename S, typename U, int V, int L, bool TORCH_LERP>
+__global__ __launch_bounds__(256) void k_state_step_narrow(const StepArgs<S, U> a) {
+  constexpr int WAYS = 16, P = WAYS * L, RW = 64 / P, UNR = 4;
+  const uint32_t wave = blockIdx.x * 4u + (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int q = lane % P, way = q / L;
+  const uint32_t row = wave * RW + (uint32_t)(lane / P);
+  const bool has_row = row < (uint32_t)a.nrows;
+  const uint32_t crow = has_row ? row : (uint32_t)a.nrows - 1;   // lanes past the step's rows read the last row's
+  const int64_t col = (int64_t)(q % L) * V;
+  // the column this lane finishes, and whether it does (the other ways of the same column hold copies)
+  const int64_t mine = col + way / (16 / V);
+  const bool active = has_row && way % (16 / V) == 0 && mine < a.batch;
+  const bool mat = a.xprev != nullptr && a.rowptr != nullptr;
+  int32_t beg = 0, end = 0;
+  if (mat) {
+    beg = a.rowptr[crow];
+    end = a.rowptr[crow + 1];
+  }
+  RowInputs<S, U, 1> in;
+  in.p = a.params[crow];
+  float acc[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) acc[i] = 0.0f;
+  const int32_t n = has_row ? end - beg : 0;
+  int32_t len = n;   // the wave's longest row
+  if constexpr (RW >= 2) len = max(len, __shfl_xor(len, 32));
+  if constexpr (RW >= 4) len = max(len, __shfl_xor(len, 16));
+  len = __builtin_amdgcn_readfirstlane(len);
+  const __amdgpu_buffer_rsrc_t r = buffer_of(a.xprev, a.xbytes);
+  const uint32_t row_bytes = (uint32_t)a.ldx * (uint32_t)sizeof(S), voff = (uint32_t)col * (uint32_t)sizeof(S);
+  // this way's records of rounds k .. k + 3 (16 non-zeros a round), the rounds no row of the wave reaches left out;
+  // lanes past their row's end load nothing, and gather nothing
+  auto records = [&](int32_t k, int2 (&rec)[UNR]) {
+#pragma unroll
+    for (int j = 0; j < UNR; ++j) {
+      const int32_t e = k + WAYS * j + way;
+      rec[j] = make_int2(0, 0);
+      if (e < n) rec[j] = a.colval[beg + e];
+    }
+  };
+  int2 rec[UNR];
+  records(0, rec);
+  load_row_drive(a, mine, active, in);
+  for (int32_t k = 0; k < len; k += WAYS * UNR) {
+    typename Lanes<S, V>::vec xr[UNR];
+#pragma unroll
+    for (int j = 0; j < UNR; ++j) {
+      xr[j] = Lanes<S, V>::zero();
+      if (k + WAYS * j + way < n) xr[j] = bload<S, V>(r, (int)(__umul24((uint32_t)rec[j].x, row_bytes) + voff), 0);
+    }
+    int2 nx[UNR];
+    records(k + WAYS * UNR, nx);
+#pragma unroll
+    for (int j = 0; j < UNR; ++j) {
+      const float wt = __int_as_float(rec[j].y);
+#pragma unroll
+      for (int i = 0; i < V; ++i) acc[i] = fmaf(wt, Lanes<S, V>::at(xr[j], i), acc[i]);
+    }
+#pragma unroll
+    for (int j = 0; j < UNR; ++j) rec[j] = nx[j];
+  }
+  const float sum[1] = {len > 0 ? narrow_sum<8 * L, L, V>(acc, lane) : 0.0f};
+  if (!active) return;
+  finish_row<S, U, 1, TORCH_LERP>(a, row, mine, sum, in);
+}
+
+// The sums of a long-row step of 1 or 2 columns (NC), from source rows staged in LDS.  Every gather from the L2 costs a
+// 128-byte line whatever it uses of it, and so small a state fits the workgroups' LDS in a few bands: workgroup
+// (row block, band) reads its band of X_{t-1} (NC * sizeof(S) bytes a row) into LDS once, in whole lines, and takes its
+// rows' records of that band (StageTables) in order, 16 lanes per row.  It stores each row's sum over the band to
+// partials (bands, nrows, NC); k_stage_finish adds a row's bands.  What is left is the record stream from HBM: 10.5M
+// non-zeros (84 MB) of a half column in 31 us and 5 us for the finish, against 73 us in the narrow kernel and 110 in
+// the swept one.  The bands of a row block run on one XCD (workgroup b
+// on XCD b mod 8), whose L2 then reads the records' lines once.
+template <typename S, int NC>
+__global__ __launch_bounds__(1024) void k_stage_sums(const int32_t *__restrict__ start, const int2 *__restrict__ colval,
+                                                     const S *__restrict__ xprev, int32_t prev_rows, int32_t nrows,
+                                                     int32_t bands, int32_t band_rows, float *__restrict__ partials) {
+  constexpr int kRowBytes = NC * (int)sizeof(S), kVecs = kStageBytes / 16 / 1024;
+  static_assert((kRowBytes == 2 || kRowBytes == 4) && kStageBytes % (16 * 1024) == 0, "rows of 2 or 4 bytes");
+  __shared__ __attribute__((aligned(16))) char stage[kStageBytes];
+  const int per = (int)(gridDim.x >> 3) / bands, slot = (int)(blockIdx.x >> 3);
+  if (slot >= per * bands) return;   // the whole workgroup
+  const int band = slot % bands, block = (int)(blockIdx.x & 7) * per + slot / bands, blocks = 8 * per;
+  const int32_t base = band * band_rows, have = min(band_rows, prev_rows - base);
+  {
+    const char *src = reinterpret_cast<const char *>(xprev) + (int64_t)base * kRowBytes;
+    const int bytes = have * kRowBytes, vecs = bytes / 16;
+    uint4 v[kVecs];   // loads without branches, all in flight together (a band holds thousands of pieces)
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i) v[i] = reinterpret_cast<const uint4 *>(src)[min(i * 1024 + (int)threadIdx.x, vecs - 1)];
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i) {
+      const int p = i * 1024 + (int)threadIdx.x;
+      if (p < vecs) reinterpret_cast<uint4 *>(stage)[p] = v[i];
+    }
+    const int p = vecs * 8 + (int)threadIdx.x;   // what is left of the last piece, 2 bytes a thread
+    if (2 * p < bytes) reinterpret_cast<uint16_t *>(stage)[p] = reinterpret_cast<const uint16_t *>(src)[p];
+  }
+  if (threadIdx.x < NC) reinterpret_cast<S *>(stage)[have * NC + threadIdx.x] = static_cast<S>(0.0f);
+  __syncthreads();
+  // A unit of 16 lanes takes 4 consecutive rows at a time, every units-th quad of the step's rows: rows of like length
+  // that sit together spread over the workgroups.
+  const int s = threadIdx.x & 15;
+  const int32_t quads = (nrows + 3) / 4, step = 64 * blocks;
+  const int32_t *from = start + (int64_t)band * nrows;
+  // lanes 0 .. 3: where the band begins in the quad's rows, lanes 4 .. 7: where it ends (loaded without a branch)
+  auto bounds = [&](int32_t quad) {
+    const int32_t r = 4 * quad + (s & 3), at = from[(s & 4 ? nrows : 0) + min(r, nrows - 1)];
+    return r < nrows ? at : 0;
+  };
+  struct Quad {
+    int32_t b[4], e[4];
+    int2 rec[4][2];
+  };
+  // the quad's bounds, and the first two rounds' records of each row (past the row's band its last record, dropped)
+  auto fetch = [&](int32_t be, Quad &w) {
+    static_for<4>([&](auto J) {
+      constexpr int j = decltype(J)::value;
+      w.b[j] = group_bcast<16, j>(be);
+      w.e[j] = group_bcast<16, j + 4>(be);
+#pragma unroll
+      for (int k = 0; k < 2; ++k) w.rec[j][k] = colval[max(min(w.b[j] + 16 * k + s, w.e[j] - 1), 0)];
+    });
+  };
+  // past the row's band: the row of zeros, with weight 0
+  auto add = [&](const int2 &rc, bool live, float (&sum)[NC]) {
+    const auto x = reinterpret_cast<const typename Lanes<S, NC>::vec *>(stage)[live ? rc.x - base : have];
+    const float wt = live ? __int_as_float(rc.y) : 0.0f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) sum[c] = fmaf(wt, Lanes<S, NC>::at(x, c), sum[c]);
+  };
+  // the quad's sums, row s >> 2 of it in lane s: stored, or added to what an earlier call stored
+  auto store = [&](int32_t quad, const float (&acc)[NC][4], bool more) {
+    float total[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) total[c] = narrow_sum<8, 1, 4>(acc[c], s);
+    const int32_t row = 4 * quad + (s >> 2);
+    if ((s & 3) == 0 && row < nrows) {
+      float *dst = partials + ((int64_t)band * nrows + row) * NC;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) dst[c] = more ? dst[c] + total[c] : total[c];
+    }
+  };
+  const int32_t first = (int32_t)(threadIdx.x >> 4) * blocks + block;
+  // Vector memory counters retire in order: the bounds of the quad after next are asked for before the next quad's
+  // records, so waiting for them leaves those records in flight while this quad is summed.  Quads past the step's rows
+  // have empty rows.
+  Quad cur;
+  fetch(bounds(first), cur);
+  int32_t be = bounds(first + step);
+  uint64_t longer = 0;   // quads with a row of more than two rounds in the band, for the pass below
+  for (int32_t quad = first, i = 0; quad < quads; quad += step, ++i) {
+    const int32_t after = bounds(quad + 2 * step);
+    Quad nxt;
+    fetch(be, nxt);
+    be = after;
+    float acc[NC][4];
+    bool more = false;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float sum[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) sum[c] = 0.0f;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) add(cur.rec[j][k], cur.b[j] + 16 * k + s < cur.e[j], sum);
+      more |= cur.e[j] - cur.b[j] > 32;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) acc[c][j] = sum[c];
+    }
+    store(quad, acc, false);
+    longer |= (uint64_t)(more ? 1 : 0) << i;
+    cur = nxt;
+  }
+  // rows of more than two rounds (a hub's thousands of records among them): 8 rounds' records at once
+  for (int32_t quad = first; longer != 0; quad += step, longer >>= 1) {
+    if (!(longer & 1)) continue;
+    const int32_t at = bounds(quad);
+    float acc[NC][4];
+    static_for<4>([&](auto J) {
+      constexpr int j = decltype(J)::value;
+      const int32_t b = group_bcast<16, j>(at), e = group_bcast<16, j + 4>(at);
+      float sum[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) sum[c] = 0.0f;
+      for (int32_t q0 = b + 32 + s; q0 < e; q0 += 8 * 16) {
+        int2 rc[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) rc[k] = colval[min(q0 + 16 * k, e - 1)];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) add(rc[k], q0 + 16 * k < e, sum);
+      }
+#pragma unroll
+      for (int c = 0; c < NC; ++c) acc[c][j] = sum[c];
+    });
+    store(quad, acc, true);
+  }
+}
+
+// A staged step's rows: the bands' sums added in band order, then the row's epilogue.  One thread per value.
+template <typename S, typename U, int NC, bool TORCH_LERP>
+__global__ __launch_bounds__(256) void k_stage_finish(const StepArgs<S, U> a, int32_t bands) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x, row = i / NC;
+  if (row >= (uint32_t)a.nrows) return;
+  const int64_t col = i % NC;
+  if (col >= a.batch) return;
+  RowInputs<S, U, 1> in;
+  load_row_inputs<S, U, 1>(a, row, col, true, in);
+  float sum[1] = {0.0f};
+  for (int32_t k = 0; k < bands; ++k) sum[0] += a.partials[(int64_t)k * a.nrows * NC + i];
+  finish_row<S, U, 1, TORCH_LERP>(a, row, col, sum, in);
 }
 
 // ---- banded sweep of the long-row steps ---------------------------------------------------------------

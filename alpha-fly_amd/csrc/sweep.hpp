@@ -46,6 +46,16 @@ struct SweepConfig {
   bool operator==(const SweepConfig &o) const { return std::memcmp(this, &o, sizeof(*this)) == 0; }
 };
 
+// Where each row's records of each band of source rows begin, for the staged step: band b holds the source rows
+// [b * band_rows, (b + 1) * band_rows), one band's state rows of 2 or 4 bytes and one row of zeros filling the LDS of a
+// workgroup.
+constexpr int kStageBytes = 144 * 1024, kStageBands = 8;
+struct StageTables {
+  int32_t bands = 0;         // 0: the structure is not staged (more than kStageBands bands, or columns out of order)
+  int32_t band_rows = 0;
+  DevArray<int32_t> start;   // (bands + 1, nrows)
+};
+
 struct SweepTables {
   int32_t bands = kSweepBands, paired = 0, grid = 0, rows_per_wave = 0;
   int32_t dealt = 0;                // the initial order was dealt out by work (the index order was unbalanced)
@@ -57,6 +67,7 @@ struct SweepTables {
   DevArray<int32_t> split;          // (split_rows): the rows split into pieces
   DevArray<int32_t> split_ptr;      // (split_rows + 1): the pieces of split[h] are split_ptr[h] .. split_ptr[h + 1] - 1
   DevArray<int32_t> piece_row;      // (pieces): the row each piece belongs to
+  StageTables stage[2];             // for state rows of 2 and of 4 bytes
 };
 
 // The GPU's CU count (the swept kernel runs one workgroup per CU), per device, cached; safe to call from several
@@ -114,6 +125,32 @@ __global__ __launch_bounds__(256) void k_band_off(const int32_t *__restrict__ ro
     o += cnt[k];
   }
   off[i * (K + 1) + K] = end;
+}
+
+// start (bands + 1, nr): the row's start plus the count of its columns below b * band_rows, by bisection; bad is raised
+// where a row's columns do not rise or leave [0, ncols).  16 lanes per row: all check, lane b searches boundary b.
+template <typename C>
+__global__ __launch_bounds__(256) void k_stage_starts(const int32_t *__restrict__ rowptr, const C *__restrict__ colval,
+                                                      int64_t nr, int64_t ncols, int32_t bands, int32_t band_rows,
+                                                      int32_t *__restrict__ start, int32_t *__restrict__ bad) {
+  const int s = threadIdx.x & 15;
+  const int64_t i = blockIdx.x * 16 + (threadIdx.x >> 4);
+  if (i >= nr) return;
+  const int32_t beg = rowptr[i], end = rowptr[i + 1];
+  bool wrong = false;
+  for (int32_t q = beg + s; q < end; q += 16) {
+    const int32_t c = record_col(colval[q]);
+    wrong |= c < 0 || c >= ncols || (q + 1 < end && c > record_col(colval[q + 1]));
+  }
+  if (wrong) atomicOr(bad, 1);
+  if (s > bands) return;
+  int32_t lo = beg, hi = s == bands ? beg : end;   // the first record at or past the boundary lies in [lo, hi]
+  while (lo < hi) {
+    const int32_t mid = lo + (hi - lo) / 2;
+    if ((int64_t)record_col(colval[mid]) < (int64_t)s * band_rows) lo = mid + 1;
+    else hi = mid;
+  }
+  start[(int64_t)s * nr + i] = s == bands ? end : lo;
 }
 
 // The order in which the swept kernel's waves take a step's rows: each wave's own `per` consecutive positions of the
@@ -442,6 +479,33 @@ __global__ void k_sweep_ranges(const int32_t *__restrict__ off, int K, int64_t n
   }
 }
 
+// The staged step's tables of t's structure: none where its columns are out of order.
+template <typename C>
+void build_stage(const int32_t *rowptr, const C *cols, SweepTables &t, hipStream_t st) {
+  DevArray<int32_t> bad(1);
+  const int32_t zero = 0;
+  FLY_HIP(hipMemcpyAsync(bad.p, &zero, sizeof(zero), hipMemcpyHostToDevice, st));
+  for (int i = 0; i < 2; ++i) {
+    const int64_t most = (kStageBytes / (2 << i) - 1) / 64 * 64, bands = (t.ncols + most - 1) / most;
+    if (bands > kStageBands) continue;
+    StageTables &s = t.stage[i];
+    s.bands = (int32_t)bands;
+    s.band_rows = (int32_t)round_up((t.ncols + bands - 1) / bands, 64);   // 64 rows: every band starts on a line
+    s.start.alloc((size_t)(bands + 1) * t.nrows);
+    hipLaunchKernelGGL(k_stage_starts<C>, dim3(blocks_for(t.nrows, 16)), dim3(256), 0, st, rowptr, cols, t.nrows,
+                       t.ncols, s.bands, s.band_rows, s.start.p, bad.p);
+  }
+  check_launch("stage tables");
+  int32_t wrong = 0;
+  FLY_HIP(hipMemcpyAsync(&wrong, bad.p, sizeof(wrong), hipMemcpyDeviceToHost, st));
+  FLY_HIP(hipStreamSynchronize(st));
+  if (!wrong) return;
+  for (StageTables &s : t.stage) {
+    s.bands = 0;
+    s.start.release();
+  }
+}
+
 }  // namespace
 
 // The tables of one CSR structure (rowptr nrows + 1, records or columns nnz, columns below ncols), or null when it
@@ -630,6 +694,7 @@ std::shared_ptr<SweepTables> build_sweep(const int32_t *rowptr, const C *cols, i
     check_launch("sweep order");
     FLY_HIP(hipStreamSynchronize(st));
   }
+  build_stage<C>(rowptr, cols, *t, st);
   FLY_HIP(hipStreamSynchronize(st));
   return t;
 }

@@ -1,0 +1,64 @@
+"""GPU parity of the small-batch state step against the CPU oracle: the narrow kernel at every width of its rows (2, 4, 16
+and 32 bytes, and the first batches past them), and the staged sums of long-row steps on a graph just past the size rule,
+with rows of no partner, of one more than two rounds of 16, and hubs.
+
+Tolerances as in test_gpu_sweep.py: float32 within float32 round-off of the float64 oracle (2e-5); the float16 state within
+2e-3 of the deviation's own scale, or 4e-3 of the largest activity where it holds the activity itself (six float16
+roundings of the state and its sum per step)."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import brain_arrays, random_params
+from test_gpu_sweep import _forward_io_both, _heavy_tailed, _rnn
+
+from oracle import forward as F
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("batch", [1, 2, 3, 4, 8, 9, 16, 17, 32, 33])
+def test_narrow_batches_match_the_oracle(batch):
+    conn = _heavy_tailed(3)
+    lg, b, al = random_params(conn, 9, gain_sd=0.1)
+    rnn = _rnn(conn, 4.0, lg, b, al)
+    ba = brain_arrays(conn, 4.0, lg, b, al, dtype=torch.float64)
+    _forward_io_both(rnn, conn, ba, batch, 6, 200 + batch, "auto")
+    u = torch.randn(conn.n_neurons, batch, generator=torch.Generator().manual_seed(batch))
+    with torch.no_grad():
+        h = rnn(u.clone().to(DEV), 4)
+    ref = F.literal(ba, u.double(), 4).numpy()
+    np.testing.assert_allclose(h.cpu().numpy(), ref, rtol=2e-5, atol=2e-5 * np.abs(ref).max())
+
+
+@pytest.fixture(scope="module")
+def staged_net():
+    """70,001 neurons (no multiple of a row quad) of 36 partners on average: enough rows, sources and partners to be
+    staged.  The first and last rows are empty, some hold 33, 96 and 97 partners and three are hubs of thousands."""
+    from chessfly.synthetic import degree_connectome
+    n = 70_001
+    rng = np.random.default_rng(5)
+    deg = rng.poisson(36, n)
+    deg[[0, 1, n - 1]] = 0
+    deg[10:14] = [33, 96, 97, 129]
+    deg[[5, 40_000, n - 2]] = [20_000, 9_193, 3_000]
+    ids = rng.permutation(n)
+    conn = degree_connectome(deg, np.sort(ids[:500]), np.sort(ids[500:700]), seed=6)
+    lg, b, al = random_params(conn, 4, gain_sd=0.1)
+    return conn, _rnn(conn, 4.0, lg, b, al), brain_arrays(conn, 4.0, lg, b, al, dtype=torch.float64)
+
+
+@pytest.mark.parametrize("batch,dtype", [(1, torch.float32), (1, torch.float16), (2, torch.float16)])
+def test_staged_steps_match_the_oracle(staged_net, batch, dtype):
+    conn, rnn, ba = staged_net
+    u = torch.randn(conn.n_neurons, batch, generator=torch.Generator().manual_seed(batch)).to(dtype)
+    with torch.no_grad():
+        h = rnn(u.clone().to(DEV), 3)
+    ref = F.literal(ba, u.double(), 3).numpy()
+    tol = 2e-5 if dtype == torch.float32 else 4e-3
+    np.testing.assert_allclose(h.double().cpu().numpy(), ref, rtol=0, atol=tol * np.abs(ref).max())
