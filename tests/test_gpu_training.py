@@ -708,3 +708,39 @@ def test_full_scale_train_step_gradients_match_the_oracle(full_net, batch):
     for name in got:
         assert float(want[name].abs().max()) > 0, name
         _close(got[name], want[name], 1e-3, name)
+
+
+@pytest.mark.parametrize("batch", [1, 3, 66, 201])
+@pytest.mark.parametrize("swept", [False, True])
+def test_cone_gradients_of_ragged_batches_match_the_oracle(batch, swept):
+    """forward_io under autograd at batches that are not a multiple of 4, which run with columns of zeros behind them:
+    outputs and gradients against the oracle in float64, in one chunk and with a ragged last one, and with the sweep
+    forced; the gradient of u_in has the batch's own shape."""
+    from chessfly import _hip
+    from chessfly.synthetic import GraphSpec, synthetic_connectome
+    from oracle import training as T
+    from oracle.lightcone import light_cone
+    conn = synthetic_connectome(GraphSpec(n=3000, edges=120_000, n_sensory=300, n_output=100, seed=5))
+    rnn, b = _rnn_pair(conn, 6)
+    rng = np.random.default_rng(batch)
+    u_in = rng.normal(0, 1, (300, batch))
+    target = torch.as_tensor(rng.normal(0, 1, (100, batch)))
+    keys = {"swept": 1, "sweep_grid": 4} if swept else {}
+    for k, v in keys.items():
+        _hip.set_tuning(k, v)
+    try:
+        u_d = torch.tensor(u_in, dtype=torch.float32, device=DEV, requires_grad=True)
+        out = rnn.forward_io(u_d, torch.arange(0, 300, device=DEV), torch.arange(2900, 3000, device=DEV), 6)
+        ((out - target.float().to(DEV)) ** 2).sum().backward()
+    finally:
+        for k in keys:
+            _hip.set_tuning(k, 0)
+    cone = light_cone(conn.n_neurons, conn.pre.numpy(), conn.post.numpy(), np.arange(300), np.arange(2900, 3000), 6)
+    u_r = torch.tensor(u_in, requires_grad=True)
+    ref = T.cone_grad(b, cone, u_r)
+    ((ref - target) ** 2).sum().backward()
+    want = [ref.detach(), u_r.grad, b.log_gain.grad, b.bias.grad, b.alpha_logit.grad]
+    got = [out.detach()] + _device_grads(rnn, u_d)
+    for g, r, name in zip(got, want, ("out", "u_in", "log_gain", "bias", "alpha_logit")):
+        assert g.shape == r.shape, name
+        _close(g, r, 1e-4, f"ragged B={batch} swept={swept} {name}")
