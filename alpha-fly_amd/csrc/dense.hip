@@ -46,7 +46,7 @@ struct fly_dense {
   fly::DevArray<float> enc_b, head_b, norm_mean, norm_var;
   fly::DevArray<int32_t> move_from, move_to;
   float enc_unscale = 1.f, head_unscale = 1.f, eps = 1e-8f, clip = 8.f;
-  int gemm_tile = 0;   // the gemm_tile tuning when the dense plan was created
+  int gemm_tile = 0, gemm_splits = 0;   // the tuning when the dense plan was created
   int64_t head_rows() const { return n_moves + 131; }
 };
 
@@ -156,6 +156,7 @@ struct Split {
 // quarter of its time.
 struct EncoderEpilogue {
   static constexpr bool kRows = true;
+  __device__ __forceinline__ EncoderEpilogue part(int) const { return *this; }   // its K loop is never split
   const float *bias;
   float gain;
   float *u;
@@ -183,11 +184,13 @@ struct EncoderEpilogue {
   }
 };
 
-// ct[n, m] = C[m, n]: one row of all head outputs per board (measured: its element stores cost about 4 us).
+// ct[n, m] = C[m, n]: one row of all head outputs per board (measured: its element stores cost about 4 us), for each
+// part of a split K loop one after the other.
 struct HeadEpilogue {
   static constexpr bool kRows = false;
   float *ct;
-  int64_t ldc;
+  int64_t ldc, part_stride;
+  __device__ __forceinline__ HeadEpilogue part(int p) const { return {ct + p * part_stride, ldc, part_stride}; }
   __device__ __forceinline__ void operator()(int64_t m, int64_t n, float v) const { ct[n * ldc + m] = v; }
   __device__ __forceinline__ void row4(int64_t, int64_t, float4, int64_t) const {}
 };
@@ -204,15 +207,15 @@ __device__ __forceinline__ void xcd_tile(int tiles, int gx, int &ty, int &tx) {
   tx = q - ty * gx;
 }
 
-// C = A B^T on split operands.  4 waves in 2 x 2, each owning (16 TM) x (16 TN) of the (32 TM) x (32 TN) tile.
+// C = A B^T over K in [kbeg, kend) on split operands.  4 waves in 2 x 2, each owning (16 TM) x (16 TN) of the (32 TM) x (32 TN) tile.
 // K is staged 64 at a time through LDS: each row of a stage is one 128-byte line, loaded by 8 consecutive lanes and
 // written to LDS in one piece; rows are padded to 144 bytes so 16-byte fragment reads are free of bank conflicts.  The
 // next stage's global loads are issued before the current stage's MFMAs.  BLO = false leaves out A_hi B_lo, for tiles
 // whose B rows are all exact in float16.
 template <int TM, int TN, bool BLO, class EP>
-__device__ __forceinline__ void gemm_tile(const Split &A, const Split &B, int64_t kp, float unscale, const EP &ep,
-                                          int64_t m0, int64_t n0, _Float16 (*As)[32 * TM][LDK],
-                                          _Float16 (*Bs)[32 * TN][LDK]) {
+__device__ __forceinline__ void gemm_tile(const Split &A, const Split &B, int64_t kp, int64_t kbeg, int64_t kend,
+                                          float unscale, const EP &ep, int64_t m0, int64_t n0,
+                                          _Float16 (*As)[32 * TM][LDK], _Float16 (*Bs)[32 * TN][LDK]) {
   constexpr int OCT = GBK / 8, RPP = 256 / OCT;          // 16-byte pieces per row, rows per pass of 256 threads
   constexpr int AL = 32 * TM / RPP, BL = 32 * TN / RPP;  // passes per operand half
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -250,8 +253,8 @@ __device__ __forceinline__ void gemm_tile(const Split &A, const Split &B, int64_
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
   const int fk = 8 * (lane >> 4), fr = lane & 15;
-  fetch(0);
-  for (int64_t k0 = 0; k0 < kp; k0 += GBK) {
+  fetch(kbeg);
+  for (int64_t k0 = kbeg; k0 < kend; k0 += GBK) {
 #pragma unroll
     for (int i = 0; i < AL; ++i) {
       *reinterpret_cast<half8 *>(&As[0][lr + RPP * i][lk]) = rah[i];
@@ -263,7 +266,7 @@ __device__ __forceinline__ void gemm_tile(const Split &A, const Split &B, int64_
       if (BLO) *reinterpret_cast<half8 *>(&Bs[1][lr + RPP * i][lk]) = rbl[i];
     }
     __syncthreads();
-    if (k0 + GBK < kp) fetch(k0 + GBK);
+    if (k0 + GBK < kend) fetch(k0 + GBK);
 #pragma unroll
     for (int kk = 0; kk < GBK; kk += 32) {
       half8 bh[TN], bl[TN];
@@ -320,9 +323,10 @@ __device__ __forceinline__ void gemm_tile(const Split &A, const Split &B, int64_
   }
 }
 
+// Tiles go by (A-tile, part of K, B-tile), so the workgroups an XCD runs together still share their A rows.
 template <int TM, int TN, class EP>
-__global__ __launch_bounds__(256) void k_gemm_split(const Split A, const Split B, int64_t kp, float unscale, const EP ep,
-                                                    int tiles, int gx) {
+__global__ __launch_bounds__(256) void k_gemm_split(const Split A, const Split B, int64_t kp, float unscale,
+                                                    const EP whole, int tiles, int gx, int splits) {
   // one block of LDS for both operands' stages and, after the K loop, the C tile of a row-wise epilogue (rows
   // padded by 4 floats)
   constexpr size_t kStages = 2 * LDK * 32 * (TM + TN);
@@ -331,7 +335,11 @@ __global__ __launch_bounds__(256) void k_gemm_split(const Split A, const Split B
   auto As = reinterpret_cast<_Float16 (*)[32 * TM][LDK]>(smem);
   auto Bs = reinterpret_cast<_Float16 (*)[32 * TN][LDK]>(smem + 2 * LDK * 32 * TM);
   int ty, tx;
-  xcd_tile(tiles, gx, ty, tx);
+  xcd_tile(tiles, gx * splits, ty, tx);
+  const int part = tx / gx;
+  tx -= part * gx;
+  const EP ep = whole.part(part);
+  const int64_t stages = kp / GBK, kbeg = stages * part / splits * GBK, kend = stages * (part + 1) / splits * GBK;
   const int64_t m0 = (int64_t)ty * (32 * TM), n0 = (int64_t)tx * (32 * TN);
   bool blo = true;
   if (B.flag != nullptr) {  // uniform over the workgroup
@@ -339,36 +347,53 @@ __global__ __launch_bounds__(256) void k_gemm_split(const Split A, const Split B
     blo = __syncthreads_or(i < 32 * TN && n0 + i < B.rows && B.flag[n0 + i] != 0);
   }
   if (blo)
-    gemm_tile<TM, TN, true>(A, B, kp, unscale, ep, m0, n0, As, Bs);
+    gemm_tile<TM, TN, true>(A, B, kp, kbeg, kend, unscale, ep, m0, n0, As, Bs);
   else
-    gemm_tile<TM, TN, false>(A, B, kp, unscale, ep, m0, n0, As, Bs);
+    gemm_tile<TM, TN, false>(A, B, kp, kbeg, kend, unscale, ep, m0, n0, As, Bs);
 }
 
-// Wave tiles of 64 x 64 (128 x 128 per workgroup) where that gives at least four tiles per CU, else 32 x 32 or
-// 32 x 80 (64 x 64 or 64 x 160 per workgroup): measured on the 17,937 x 1120 encoder and the 4,299 x 1120 head.
-// The gemm_tile tuning key forces one: 1 = 64 x 64, 2 = 128 x 64, 3 = 128 x 128, or 10 TM + TN for a workgroup tile
-// of 32 TM x 32 TN with TM in {2, 3, 4} and TN in {2, 4, 5}.
-template <class EP>
-void gemm_split(const Split &A, const Split &B, int64_t kp, float unscale, const EP &ep, int tile_key,
-                hipStream_t st) {
-  if (A.rows == 0 || B.rows == 0) return;
-  auto count = [&](int bm, int bn) { return ((A.rows + bm - 1) / bm) * ((B.rows + bn - 1) / bn); };
+// The workgroup tile, 10 TM + TN for 32 TM x 32 TN.  The gemm_tile tuning key forces one: 1 = 64 x 64, 2 = 128 x 64,
+// 3 = 128 x 128, or 10 TM + TN with TM in {2, 3, 4} and TN in {2, 4, 5}.  Otherwise, measured on the 17,937-row encoder
+// and the 4,299-row head (us):
+// * 128 x 128 from 1,024 tiles on: encoder of 1120 boards 106 against 121 (64 x 64) and 112 (64 x 160);
+// * 64 x 160 where its columns cover the batch with no more padding than 64 do and its tiles fill at least 82% of their
+//   rounds of 512 workgroups (two per CU): head of 1120 boards 125 against 129 (64 x 64), encoder of 480 60 against 68;
+//   with rounds less full it loses (head of 640: 103 against 87, of 1280: 167 against 147);
+// * 128 x 128 from 400 tiles on that pad at most 10% more columns than 64: head of 1500 boards 154 against 169, encoder
+//   of 640 73 against 77, but of 400 (512 columns against 448) 65 against 60;
+// * else 64 x 64.
+int gemm_shape(int64_t arows, int64_t brows, int tile_key) {
   int shape = tile_key;
   if (shape == 1) shape = 22;
   else if (shape == 2) shape = 42;
   else if (shape == 3) shape = 44;
   const int tm = shape / 10, tn = shape % 10;
-  const bool known = (tm == 2 || tm == 3 || tm == 4) && (tn == 2 || tn == 4 || tn == 5);
-  // smaller GEMMs (the head): 64 x 160 where 160-column tiles cover the batch with no more padding than 64-column
-  // ones (B = 1120: 7 tiles against 17.5, one round of workgroups; 6 us faster), else 64 x 64
-  if (!known) shape = count(128, 128) >= 1024 ? 44 : (round_up(B.rows, 160) <= round_up(B.rows, 64) ? 25 : 22);
+  if ((tm == 2 || tm == 3 || tm == 4) && (tn == 2 || tn == 4 || tn == 5)) return shape;
+  const int64_t large = ((arows + 127) / 128) * ((brows + 127) / 128);
+  if (large >= 1024) return 44;
+  const int64_t wide = ((arows + 63) / 64) * ((brows + 159) / 160);
+  if (round_up(brows, 160) <= round_up(brows, 64) && wide * 100 >= round_up(wide, 512) * 82) return 25;
+  return large >= 400 && round_up(brows, 128) * 10 <= round_up(brows, 64) * 11 ? 44 : 22;
+}
+
+int64_t gemm_tiles(int64_t arows, int64_t brows, int shape) {
   const int bm = 32 * (shape / 10), bn = 32 * (shape % 10);
-  const int64_t gx = (B.rows + bn - 1) / bn, tiles = count(bm, bn);
+  return ((arows + bm - 1) / bm) * ((brows + bn - 1) / bn);
+}
+
+template <class EP>
+void gemm_split(const Split &A, const Split &B, int64_t kp, float unscale, const EP &ep, int tile_key, int splits,
+                hipStream_t st) {
+  if (A.rows == 0 || B.rows == 0) return;
+  const int shape = gemm_shape(A.rows, B.rows, tile_key);
+  const int bn = 32 * (shape % 10);
+  const int64_t gx = (B.rows + bn - 1) / bn, tiles = gemm_tiles(A.rows, B.rows, shape) * splits;
   FLY_REQUIRE(tiles < INT32_MAX, "GEMM grid too large");
   const dim3 grid((unsigned)tiles), block(256);
 #define FLY_GEMM_CASE(TM_, TN_)                                                                                    \
   case 10 * TM_ + TN_:                                                                                             \
-    hipLaunchKernelGGL((k_gemm_split<TM_, TN_, EP>), grid, block, 0, st, A, B, kp, unscale, ep, (int)tiles, (int)gx); \
+    hipLaunchKernelGGL((k_gemm_split<TM_, TN_, EP>), grid, block, 0, st, A, B, kp, unscale, ep, (int)tiles, (int)gx, \
+                       splits);                                                                                     \
     break;
   switch (shape) {
     FLY_GEMM_CASE(2, 2)
@@ -388,24 +413,36 @@ void gemm_split(const Split &A, const Split &B, int64_t kp, float unscale, const
 
 // logits[n, i] = (ct[n, i] + b[i]) + (ct[n, M + f] + b[M + f]) + (ct[n, M + 64 + t] + b[M + 64 + t]),
 // wdl[n, j] = ct[n, M + 128 + j] + b[M + 128 + j], with M = n_moves and (f, t) the move's squares.
+// ct holds `parts` shares of C (a split K loop's), part_stride apart, added in order.
 // One workgroup per board: its from- and to-square terms (64 + 64 values plus biases) go to LDS once, then each
 // thread writes 4 consecutive moves with 16-byte loads and stores when `vec` (the move count and the rows allow
 // them), one move at a time otherwise.
-__global__ __launch_bounds__(256) void k_assemble(const float *__restrict__ ct, int64_t ldc, int64_t n_moves,
+__global__ __launch_bounds__(256) void k_assemble(const float *__restrict__ ct, int64_t ldc, int32_t parts,
+                                                  int64_t part_stride, int64_t n_moves,
                                                   const float *__restrict__ b, const int32_t *__restrict__ mfrom,
                                                   const int32_t *__restrict__ mto, int64_t batch, bool vec,
                                                   float *__restrict__ logits, float *__restrict__ wdl) {
   __shared__ float sq[128];
   for (int64_t n = blockIdx.x; n < batch; n += gridDim.x) {
     const float *row = ct + n * ldc;
+    auto value = [&](int64_t i) {
+      float v = row[i];
+      for (int32_t p = 1; p < parts; ++p) v += row[p * part_stride + i];
+      return v;
+    };
     __syncthreads();   // the previous board's squares are read
-    if (threadIdx.x < 128) sq[threadIdx.x] = row[n_moves + threadIdx.x] + b[n_moves + threadIdx.x];
-    if (threadIdx.x < 3) wdl[n * 3 + threadIdx.x] = row[n_moves + 128 + threadIdx.x] + b[n_moves + 128 + threadIdx.x];
+    if (threadIdx.x < 128) sq[threadIdx.x] = value(n_moves + threadIdx.x) + b[n_moves + threadIdx.x];
+    if (threadIdx.x < 3) wdl[n * 3 + threadIdx.x] = value(n_moves + 128 + threadIdx.x) + b[n_moves + 128 + threadIdx.x];
     __syncthreads();
     float *out = logits + n * n_moves;
     if (vec) {
       for (int64_t i = 4 * (int64_t)threadIdx.x; i < n_moves; i += 4 * (int64_t)blockDim.x) {
-        const float4 p = *reinterpret_cast<const float4 *>(row + i), bp = *reinterpret_cast<const float4 *>(b + i);
+        float4 p = *reinterpret_cast<const float4 *>(row + i);
+        const float4 bp = *reinterpret_cast<const float4 *>(b + i);
+        for (int32_t q = 1; q < parts; ++q) {
+          const float4 w = *reinterpret_cast<const float4 *>(row + q * part_stride + i);
+          p = make_float4(p.x + w.x, p.y + w.y, p.z + w.z, p.w + w.w);
+        }
         const int4 fr = *reinterpret_cast<const int4 *>(mfrom + i), to = *reinterpret_cast<const int4 *>(mto + i);
         *reinterpret_cast<float4 *>(out + i) =
             make_float4(((p.x + bp.x) + sq[fr.x]) + sq[64 + to.x], ((p.y + bp.y) + sq[fr.y]) + sq[64 + to.y],
@@ -413,7 +450,7 @@ __global__ __launch_bounds__(256) void k_assemble(const float *__restrict__ ct, 
       }
     } else {
       for (int64_t i = threadIdx.x; i < n_moves; i += blockDim.x)
-        out[i] = ((row[i] + b[i]) + sq[mfrom[i]]) + sq[64 + mto[i]];
+        out[i] = ((value(i) + b[i]) + sq[mfrom[i]]) + sq[64 + mto[i]];
     }
   }
 }
@@ -478,8 +515,28 @@ size_t encoder_ws(const fly_dense &d, int64_t batch) {
   return 2 * split_bytes(batch, d.kp_enc) + align256((size_t)batch * sizeof(int32_t));
 }
 
+// Parts of the head GEMM's K loop.  Its 4,299 rows make few tiles (68 for up to 64 boards), each a chain of 37 stages;
+// parts of K fill the other CUs, at the cost of a share of C each (k_assemble adds them).  The fewest parts, up to 3,
+// within 15% of the least rounds of 512 workgroups (two per CU) per part; none past 640 tiles, where the shares' bytes
+// cost what the rounds gain.  Measured, us of the head for 1, 2 and 3 parts: 1 board 42 / 30 / 27 (6: 30, 8: 34), 128
+// boards 52 / 44 / 38, 256 boards 65 / 57 / 55, 480 boards 89 / 77 / 87, 640 boards 113 / 107 / 103, 1120 boards 125 /
+// 135 / 152.
+int head_splits(const fly_dense &d, int64_t batch) {
+  const int64_t stages = d.kp_head / GBK;
+  if (d.gemm_splits > 0) return (int)std::min<int64_t>(d.gemm_splits, stages);
+  const int64_t tiles = gemm_tiles(d.head_rows(), batch, gemm_shape(d.head_rows(), batch, d.gemm_tile));
+  const int most = tiles > 640 ? 1 : (int)std::min<int64_t>(3, stages);
+  auto cost = [&](int s) { return (double)((tiles * s + 511) / 512) / s; };
+  double least = cost(1);
+  for (int s = 2; s <= most; ++s) least = std::min(least, cost(s));
+  int s = 1;
+  while (cost(s) > 1.15 * least) ++s;
+  return s;
+}
+
 size_t head_ws(const fly_dense &d, int64_t batch) {
-  return 2 * split_bytes(batch, d.kp_head) + align256((size_t)batch * head_ld(d) * sizeof(float));
+  return 2 * split_bytes(batch, d.kp_head) +
+         align256((size_t)head_splits(d, batch) * (size_t)batch * head_ld(d) * sizeof(float));
 }
 
 void run_encoder(const fly_dense &d, const void *x, bool x_f16, int64_t ldx, int64_t batch, float gain, float *u,
@@ -493,7 +550,7 @@ void run_encoder(const fly_dense &d, const void *x, bool x_f16, int64_t ldx, int
   else
     split_into(static_cast<const float *>(x), ldx, batch, d.k, 1.0f, xh, xl, d.kp_enc, st, exact);
   gemm_split(Split{d.enc_hi.p, d.enc_lo.p, d.n_in, nullptr}, Split{xh, xl, batch, exact}, d.kp_enc, d.enc_unscale,
-             EncoderEpilogue{d.enc_b.p, gain, u, u16, ldu}, d.gemm_tile, st);
+             EncoderEpilogue{d.enc_b.p, gain, u, u16, ldu}, d.gemm_tile, 1, st);
 }
 
 template <typename S>
@@ -510,11 +567,12 @@ void run_head(const fly_dense &d, const S *state, int64_t lds, const int32_t *sr
                      d.eps, d.clip, d.n_out, batch, rh, rl, d.kp_head);
   check_launch("normalised outputs");
   const int64_t ldc = head_ld(d);
+  const int splits = head_splits(d, batch);
   gemm_split(Split{d.head_hi.p, d.head_lo.p, d.head_rows(), nullptr}, Split{rh, rl, batch, nullptr}, d.kp_head,
-             d.head_unscale,
-             HeadEpilogue{ct, ldc}, d.gemm_tile, st);
+             d.head_unscale, HeadEpilogue{ct, ldc, batch * ldc}, d.gemm_tile, splits, st);
   const bool avec = d.n_moves % 4 == 0 && ldc % 4 == 0 && aligned(logits, 16);
-  hipLaunchKernelGGL(k_assemble, dim3((unsigned)std::min<int64_t>(batch, 65535)), dim3(256), 0, st, ct, ldc, d.n_moves,
+  hipLaunchKernelGGL(k_assemble, dim3((unsigned)std::min<int64_t>(batch, 65535)), dim3(256), 0, st, ct, ldc, splits,
+                     batch * ldc, d.n_moves,
                      d.head_b.p, d.move_from.p, d.move_to.p, batch, avec, logits, wdl);
   check_launch("head assembly");
 }
@@ -543,7 +601,9 @@ extern "C" int fly_dense_create(const fly_head_desc *h, const float *enc_w, int6
     hipStream_t st = as_stream(stream);
     auto d = std::make_unique<fly_dense>();
     d->device = current_device();
-    d->gemm_tile = tuning_snapshot().gemm_tile;
+    const Tuning tune = tuning_snapshot();
+    d->gemm_tile = tune.gemm_tile;
+    d->gemm_splits = tune.gemm_splits;
     d->n_in = n_in;
     d->k = k;
     d->kp_enc = pad_k(k);

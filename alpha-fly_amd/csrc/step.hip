@@ -709,6 +709,7 @@ const TuningKey kTuningKeys[] = {
     {"tiles", &Tuning::tiles, -kAny, kAny},
     {"spmm_groups", &Tuning::spmm_groups, -kAny, kAny},
     {"gemm_tile", &Tuning::gemm_tile, -kAny, kAny},
+    {"gemm_splits", &Tuning::gemm_splits, 0, 8},
     {"download_blocks", &Tuning::download_blocks, -kAny, kAny},
     {"swept", &Tuning::swept, -1, 1},
     {"sweep_bands", &Tuning::sweep_bands, -kAny, kAny},

@@ -481,7 +481,7 @@ int64_t fly_profile_launches(int32_t *cls, double *ms, int64_t cap);
  * half-state elements per lane of those row slots (8 = 16 bytes, 16 = 32 bytes; 0 = automatic); "spmm_groups":
  * lane groups of fly_spmm on 16-byte lanes (2, 4, 8; 0 = automatic); "gemm_tile": workgroup tile of the dense
  * maps (1 = 64 x 64, 2 = 128 x 64, 3 = 128 x 128, or 10 TM + TN for 32 TM x 32 TN with TM in {2, 3, 4} and TN in
- * {2, 4, 5}; 0 = automatic); "step_lds": bytes of LDS each state-step workgroup reserves, which caps the
+ * {2, 4, 5}; 0 = automatic); "gemm_splits": parts of the head's K loop, 1 to 8 (0 = automatic); "step_lds": bytes of LDS each state-step workgroup reserves, which caps the
  * workgroups a CU runs at once (0 = none); "download_blocks": workgroups of fly_evaluator_download when its call
  * passes 0 (0 = 16); "swept": -1 keeps the long-row steps on the grouped kernel instead of the banded sweep, 1
  * sweeps every step with a matrix whatever its size (small graphs in tests), 0 = the size rule; "sweep_bands":
