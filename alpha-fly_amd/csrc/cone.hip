@@ -269,6 +269,10 @@ void validate_graph(int64_t n, int64_t n_edges, const int32_t *crow, const int32
   int32_t h = 0;
   FLY_HIP(hipMemcpyAsync(&h, bad.p, sizeof(h), hipMemcpyDeviceToHost, st));
   FLY_HIP(hipStreamSynchronize(st));
+  {
+    QuietRelease quiet;
+    bad.release();
+  }
   FLY_REQUIRE(!(h & 2), "crow is not a CSR row pointer of n_edges edges (crow[0] == 0, non-decreasing, crow[n] == n_edges)");
   FLY_REQUIRE(!(h & 1), "pre holds a neuron id outside [0, n)");
 }
@@ -413,7 +417,9 @@ extern "C" int fly_cone_create(int64_t n, int64_t n_edges, const int32_t *crow, 
 }
 
 extern "C" int fly_cone_destroy(fly_cone *cone) {
-  return guard([&] { delete cone; });
+  return guard([&] {
+    if (cone) delete_object(cone, cone->device);
+  });
 }
 
 extern "C" int fly_cone_sizes(const fly_cone *cone, int64_t *rows, int64_t *nnz, int32_t *has_op) {

@@ -455,17 +455,31 @@ __global__ __launch_bounds__(256) void k_assemble(const float *__restrict__ ct, 
   }
 }
 
-// Grid-stride max of |w| with one atomic per wave (a fixed grid keeps the atomics on the one word few).
-__global__ void k_max_abs(const float *__restrict__ w, int64_t ld, int64_t rows, int64_t k, unsigned *__restrict__ out) {
+// max of |w| over rows x k: a wave per row in turn, four loads in flight, one atomic per workgroup (60 MB of encoder
+// weights in 18 us; one flat index per element, divided by k, took 80).
+__global__ __launch_bounds__(256) void k_max_abs(const float *__restrict__ w, int64_t ld, int64_t rows, int64_t k,
+                                                 unsigned *__restrict__ out) {
+  __shared__ float most[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   float a = 0.0f;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < rows * k; i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = i / k, c = i - r * k;
-    a = fmaxf(a, fabsf(w[r * ld + c]));
+  for (int64_t r = blockIdx.x * 4ll + wave; r < rows; r += gridDim.x * 4ll) {
+    const float *row = w + r * ld;
+    for (int64_t c = lane; c < k; c += 256) {
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = row[min(c + 64 * j, k - 1)];   // past the row's end its last element again
+#pragma unroll
+      for (int j = 0; j < 4; ++j) a = fmaxf(a, fabsf(v[j]));
+    }
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) a = fmaxf(a, __shfl_xor(a, off));
+  if (lane == 0) most[wave] = a;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  a = fmaxf(fmaxf(most[0], most[1]), fmaxf(most[2], most[3]));
   // non-negative floats order like their bit patterns
-  if ((threadIdx.x & 63) == 0 && a > 0.0f) atomicMax(out, __float_as_uint(a));
+  if (a > 0.0f) atomicMax(out, __float_as_uint(a));
 }
 
 __global__ void k_check_squares(const int32_t *__restrict__ sq, int64_t n, int32_t *__restrict__ bad) {
@@ -473,22 +487,20 @@ __global__ void k_check_squares(const int32_t *__restrict__ sq, int64_t n, int32
   if (i < n && (sq[i] < 0 || sq[i] > 63)) atomicOr(bad, 1);
 }
 
-__global__ void k_zero_u32(unsigned *__restrict__ p) { *p = 0u; }
+__global__ void k_zero_u32(unsigned *__restrict__ p) { p[threadIdx.x] = 0u; }
 
 constexpr int kThreads = 256;
 
-// Power-of-two scale that puts the largest |w| at 2^14 (low halves stay normal fp16 for every weight that
-// matters); 1 for an all-zero matrix.
-float weight_scale(const float *w, int64_t ld, int64_t rows, int64_t k, hipStream_t st) {
-  if (rows * k == 0) return 1.0f;
-  DevArray<unsigned> mx(1);
-  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, st, mx.p);
-  hipLaunchKernelGGL(k_max_abs, dim3((unsigned)std::min<int64_t>(blocks_for(rows * k, kThreads), 1024)), dim3(kThreads), 0,
-                     st, w, ld, rows, k, mx.p);
+void launch_max_abs(const float *w, int64_t ld, int64_t rows, int64_t k, unsigned *out, hipStream_t st) {
+  if (rows * k == 0) return;
+  hipLaunchKernelGGL(k_max_abs, dim3((unsigned)std::min<int64_t>(blocks_for(rows, 4), 1024)), dim3(256), 0, st, w, ld, rows,
+                     k, out);
   check_launch("max abs");
-  unsigned bits = 0;
-  FLY_HIP(hipMemcpyAsync(&bits, mx.p, sizeof(bits), hipMemcpyDeviceToHost, st));
-  FLY_HIP(hipStreamSynchronize(st));
+}
+
+// Power-of-two scale that puts the largest |w|, whose bits these are, at 2^14 (low halves stay normal fp16 for every
+// weight that matters); 1 for an all-zero matrix.
+float weight_scale(unsigned bits) {
   float m;
   memcpy(&m, &bits, sizeof(m));
   FLY_REQUIRE(std::isfinite(m), "dense weights hold a non-finite value");
@@ -612,21 +624,32 @@ extern "C" int fly_dense_create(const fly_head_desc *h, const float *enc_w, int6
     d->kp_head = pad_k(h->n_out);
     d->eps = h->norm_eps;
     d->clip = h->norm_clip;
-    {  // move squares must index the 64 from/to rows
-      DevArray<int32_t> bad(1);
-      hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, st, reinterpret_cast<unsigned *>(bad.p));
-      hipLaunchKernelGGL(k_check_squares, dim3(blocks_for(h->n_moves, kThreads)), dim3(kThreads), 0, st, h->move_from,
-                         h->n_moves, bad.p);
-      hipLaunchKernelGGL(k_check_squares, dim3(blocks_for(h->n_moves, kThreads)), dim3(kThreads), 0, st, h->move_to,
-                         h->n_moves, bad.p);
+    const int64_t K = h->n_out, M = h->n_moves;
+    struct Part {
+      const float *w, *b;
+      int64_t rows, off;
+    } parts[4] = {{h->policy_w, h->policy_b, M, 0}, {h->from_w, h->from_b, 64, M}, {h->to_w, h->to_b, 64, M + 64},
+                  {h->value_w, h->value_b, 3, M + 128}};
+    // the largest weights (encoder, then the head's parts) and whether a move's square lies outside 0..63, read back
+    // in one go
+    unsigned seen[6] = {};
+    {
+      DevArray<unsigned> found(6);
+      hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(6), 0, st, found.p);
+      launch_max_abs(enc_w, ldw, n_in, k, found.p, st);
+      for (int i = 0; i < 4; ++i) launch_max_abs(parts[i].w, K, parts[i].rows, K, found.p + 1 + i, st);
+      for (const int32_t *sq : {h->move_from, h->move_to})
+        hipLaunchKernelGGL(k_check_squares, dim3(blocks_for(M, kThreads)), dim3(kThreads), 0, st, sq, M,
+                           reinterpret_cast<int32_t *>(found.p + 5));
       check_launch("square check");
-      int32_t hb = 0;
-      FLY_HIP(hipMemcpyAsync(&hb, bad.p, sizeof(hb), hipMemcpyDeviceToHost, st));
+      FLY_HIP(hipMemcpyAsync(seen, found.p, sizeof(seen), hipMemcpyDeviceToHost, st));
       FLY_HIP(hipStreamSynchronize(st));
-      FLY_REQUIRE(hb == 0, "move_from / move_to hold a square outside 0..63");
+      QuietRelease quiet;   // used on this stream only
+      found.release();
     }
+    FLY_REQUIRE(seen[5] == 0, "move_from / move_to hold a square outside 0..63");
     // encoder
-    const float es = weight_scale(enc_w, ldw, n_in, k, st);
+    const float es = weight_scale(seen[0]);
     d->enc_unscale = 1.0f / es;
     d->enc_hi.alloc(n_in * d->kp_enc);
     d->enc_lo.alloc(n_in * d->kp_enc);
@@ -634,15 +657,9 @@ extern "C" int fly_dense_create(const fly_head_desc *h, const float *enc_w, int6
     d->enc_b.alloc(n_in);
     if (n_in) FLY_HIP(hipMemcpyAsync(d->enc_b.p, enc_b, sizeof(float) * n_in, hipMemcpyDeviceToDevice, st));
     // head: policy, from, to and value rows stacked under one scale
-    const int64_t K = h->n_out, M = h->n_moves;
-    struct Part {
-      const float *w, *b;
-      int64_t rows, off;
-    } parts[4] = {{h->policy_w, h->policy_b, M, 0}, {h->from_w, h->from_b, 64, M}, {h->to_w, h->to_b, 64, M + 64},
-                  {h->value_w, h->value_b, 3, M + 128}};
     float hs = 0.0f;
-    for (const Part &p : parts) {
-      const float s = weight_scale(p.w, K, p.rows, K, st);
+    for (int i = 0; i < 4; ++i) {
+      const float s = weight_scale(seen[1 + i]);
       hs = (hs == 0.0f) ? s : std::min(hs, s);
     }
     d->head_unscale = 1.0f / hs;
@@ -668,7 +685,9 @@ extern "C" int fly_dense_create(const fly_head_desc *h, const float *enc_w, int6
 }
 
 extern "C" int fly_dense_destroy(fly_dense *d) {
-  return guard([&] { delete d; });
+  return guard([&] {
+    if (d) delete_object(d, d->device);
+  });
 }
 
 extern "C" size_t fly_encoder_workspace(const fly_dense *d, int64_t batch) { return d ? encoder_ws(*d, batch) : 0; }

@@ -302,6 +302,8 @@ extern "C" int fly_plan_create(const fly_cone *cone, const int32_t *crow, const 
     }
     check_launch("plan");
     FLY_HIP(hipStreamSynchronize(st));
+    QuietRelease quiet;   // the temporaries were used on this stream only
+    for (DevArray<float> *tmp : {&alpha, &k_full, &c_a, &c_b}) tmp->release();
     *out = plan.release();
   });
 }
@@ -357,12 +359,16 @@ extern "C" int fly_plan_create_full(int64_t n, int64_t n_edges, const int32_t *c
     }
     check_launch("full plan");
     FLY_HIP(hipStreamSynchronize(st));
+    QuietRelease quiet;   // used on this stream only
+    alpha.release();
     *out = plan.release();
   });
 }
 
 extern "C" int fly_plan_destroy(fly_plan *plan) {
-  return guard([&] { delete plan; });
+  return guard([&] {
+    if (plan) delete_object(plan, plan->device);
+  });
 }
 
 extern "C" int fly_plan_resting(const fly_plan *plan, float *c_out, void *stream) {
@@ -411,7 +417,9 @@ extern "C" int fly_sweep_create(const int32_t *rowptr, const int32_t *col, int64
 }
 
 extern "C" int fly_sweep_destroy(fly_sweep *sweep) {
-  return guard([&] { delete sweep; });
+  return guard([&] {
+    if (sweep) delete_object(sweep, sweep->device);
+  });
 }
 
 extern "C" int fly_sweep_info(const fly_sweep *sweep, int64_t *info) {

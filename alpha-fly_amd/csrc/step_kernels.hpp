@@ -1544,7 +1544,11 @@ inline LeadSlots build_lead_slots(const int32_t *rowptr, int64_t nrows, int64_t 
   std::vector<int32_t> list;
   for (int64_t i = 0; i < slots; ++i)
     if (hf[i]) list.push_back((int32_t)i);
-  if (list.empty()) return out;
+  if (list.empty()) {
+    QuietRelease quiet;   // used on this stream only
+    flag.release();
+    return out;
+  }
   out.lead.alloc(list.size());
   FLY_HIP(hipMemcpyAsync(out.lead.p, list.data(), sizeof(int32_t) * list.size(), hipMemcpyHostToDevice, st));
   FLY_HIP(hipStreamSynchronize(st));   // the host list is a temporary
