@@ -72,30 +72,45 @@ inline int current_device() {
 // around them).  At most kMost bytes per device stay idle, and all of them go back to the runtime when the last array
 // of the process's library objects on that device is released, or when an allocation fails.
 //
-// A block is handed on only once no GPU work can still use it: release() waits for its device, as hipFree does, unless
-// a QuietRelease on this thread says that the caller has waited already.  Safe to use from several threads.
+// A block is handed on only once no GPU work can still use it: alloc() waits for the device if the block came back
+// after the last such wait, unless a QuietRelease said then that its work was over.  Releasing makes no GPU call while
+// the block stays here, so an object may go away while a stream is being captured.  Safe to use from several threads.
 class DevicePool {
  public:
   static DevicePool &get() {
     static DevicePool *pool = new DevicePool;   // never destroyed: no device memory is freed while the process exits
     return *pool;
   }
+  // `device`: the current one.
   void *alloc(size_t bytes, int device) {
     bytes = rounded(bytes);
+    void *p = nullptr;
+    bool wait = false;
+    uint64_t upto = 0;   // a wait that starts now covers the blocks that came back as number 1 .. upto
     {
       std::lock_guard<std::mutex> lock(mu_);
       Device &d = devices_[device];
       const auto best = d.idle.lower_bound(bytes);   // the smallest that holds it
       if (best != d.idle.end() && best->first <= bytes + bytes / 4) {
-        void *p = best->second;
+        p = best->second.p;
+        wait = best->second.back > d.waited;
+        upto = d.back;
         sizes_[p] = best->first;
         d.idle_bytes -= best->first;
         d.idle.erase(best);
         ++d.live;
-        return p;
       }
     }
-    void *p = nullptr;
+    if (p && wait) {
+      if (const hipError_t e = hipDeviceSynchronize(); e != hipSuccess) {
+        (void)hipGetLastError();
+        free(p, device, false);
+        FLY_HIP(e);
+      }
+      std::lock_guard<std::mutex> lock(mu_);
+      devices_[device].waited = std::max(devices_[device].waited, upto);
+    }
+    if (p) return p;
     if (hipMalloc(&p, bytes) != hipSuccess) {
       (void)hipGetLastError();
       trim(device);
@@ -106,8 +121,8 @@ class DevicePool {
     ++devices_[device].live;
     return p;
   }
-  // p: from alloc on `device`, with no GPU work left that uses it.
-  void free(void *p, int device) {
+  // p: from alloc on `device`; `quiet`: no GPU work is left that uses it.
+  void free(void *p, int device, bool quiet) {
     std::vector<void *> give;
     {
       std::lock_guard<std::mutex> lock(mu_);
@@ -116,22 +131,27 @@ class DevicePool {
       const size_t bytes = it->second;
       sizes_.erase(it);
       if (d.idle_bytes + bytes <= kMost) {
-        d.idle.emplace(bytes, p);
+        d.idle.emplace(bytes, Block{p, quiet ? 0 : ++d.back});
         d.idle_bytes += bytes;
       } else {
         give.push_back(p);
       }
       if (--d.live == 0) take_idle(d, give);
     }
-    for (void *q : give) (void)hipFree(q);
+    for (void *q : give) (void)hipFree(q);   // waits for the device itself
   }
 
  private:
   static constexpr size_t kMost = (size_t)512 << 20;
+  struct Block {
+    void *p;
+    uint64_t back;   // the how-manieth block that came back with work perhaps left; 0: without
+  };
   struct Device {
-    std::multimap<size_t, void *> idle;
+    std::multimap<size_t, Block> idle;
     size_t idle_bytes = 0;
-    int64_t live = 0;   // arrays handed out
+    uint64_t back = 0, waited = 0;   // blocks that came back so, and how many of them a wait has covered
+    int64_t live = 0;                // arrays handed out
   };
   // whole 2 MiB pages for large arrays, so the arrays of the next weight version find blocks of their own size
   static size_t rounded(size_t bytes) {
@@ -139,7 +159,7 @@ class DevicePool {
     return (bytes + unit - 1) / unit * unit;
   }
   static void take_idle(Device &d, std::vector<void *> &out) {
-    for (const auto &e : d.idle) out.push_back(e.second);
+    for (const auto &e : d.idle) out.push_back(e.second.p);
     d.idle.clear();
     d.idle_bytes = 0;
   }
@@ -170,24 +190,6 @@ class QuietRelease {
   }
 };
 
-// Waits for all work on `device`.
-inline void wait_device(int device) {
-  int cur = device;
-  (void)hipGetDevice(&cur);
-  if (cur != device) (void)hipSetDevice(device);
-  (void)hipDeviceSynchronize();
-  if (cur != device) (void)hipSetDevice(cur);
-}
-
-// Deletes an object whose arrays live on `device`, waiting for the device once for all of them.
-template <typename T>
-void delete_object(T *object, int device) {
-  if (!object) return;
-  wait_device(device);
-  QuietRelease quiet;
-  delete object;
-}
-
 // Device allocation owned by a library object, from the pool.
 template <typename T>
 struct DevArray {
@@ -212,10 +214,7 @@ struct DevArray {
     n = count;
   }
   void release() {
-    if (p) {
-      if (QuietRelease::depth() == 0) wait_device(device);
-      DevicePool::get().free(p, device);
-    }
+    if (p) DevicePool::get().free(p, device, QuietRelease::depth() > 0);
     p = nullptr;
     n = 0;
   }

@@ -417,9 +417,7 @@ extern "C" int fly_cone_create(int64_t n, int64_t n_edges, const int32_t *crow, 
 }
 
 extern "C" int fly_cone_destroy(fly_cone *cone) {
-  return guard([&] {
-    if (cone) delete_object(cone, cone->device);
-  });
+  return guard([&] { delete cone; });
 }
 
 extern "C" int fly_cone_sizes(const fly_cone *cone, int64_t *rows, int64_t *nnz, int32_t *has_op) {

@@ -685,9 +685,7 @@ extern "C" int fly_dense_create(const fly_head_desc *h, const float *enc_w, int6
 }
 
 extern "C" int fly_dense_destroy(fly_dense *d) {
-  return guard([&] {
-    if (d) delete_object(d, d->device);
-  });
+  return guard([&] { delete d; });
 }
 
 extern "C" size_t fly_encoder_workspace(const fly_dense *d, int64_t batch) { return d ? encoder_ws(*d, batch) : 0; }

@@ -366,9 +366,7 @@ extern "C" int fly_plan_create_full(int64_t n, int64_t n_edges, const int32_t *c
 }
 
 extern "C" int fly_plan_destroy(fly_plan *plan) {
-  return guard([&] {
-    if (plan) delete_object(plan, plan->device);
-  });
+  return guard([&] { delete plan; });
 }
 
 extern "C" int fly_plan_resting(const fly_plan *plan, float *c_out, void *stream) {
@@ -417,9 +415,7 @@ extern "C" int fly_sweep_create(const int32_t *rowptr, const int32_t *col, int64
 }
 
 extern "C" int fly_sweep_destroy(fly_sweep *sweep) {
-  return guard([&] {
-    if (sweep) delete_object(sweep, sweep->device);
-  });
+  return guard([&] { delete sweep; });
 }
 
 extern "C" int fly_sweep_info(const fly_sweep *sweep, int64_t *info) {
