@@ -546,9 +546,18 @@ int head_splits(const fly_dense &d, int64_t batch) {
   return s;
 }
 
+// The head's scratch with `rows` rows of C (boards times parts).
+size_t head_ws_rows(const fly_dense &d, int64_t batch, int64_t rows) {
+  return 2 * split_bytes(batch, d.kp_head) + align256((size_t)rows * head_ld(d) * sizeof(float));
+}
+
+// Room for the parts of `batch` boards and of every smaller batch (a forward's last block, or a caller that keeps one
+// workspace): head_splits may give a smaller batch more rows of C, 576 boards two parts where 640 have one.  Batches
+// with parts have up to 640 tiles and at most 1,280 with their parts (two parts of 640, three of 341), each of at most
+// 128 rows and 160 boards.
 size_t head_ws(const fly_dense &d, int64_t batch) {
-  return 2 * split_bytes(batch, d.kp_head) +
-         align256((size_t)head_splits(d, batch) * (size_t)batch * head_ld(d) * sizeof(float));
+  const int64_t most = 1280 * 160 / ((d.head_rows() + 127) / 128);
+  return head_ws_rows(d, batch, d.gemm_splits > 0 ? d.gemm_splits * batch : std::max(batch, std::min(3 * batch, most)));
 }
 
 void run_encoder(const fly_dense &d, const void *x, bool x_f16, int64_t ldx, int64_t batch, float gain, float *u,
@@ -565,9 +574,10 @@ void run_encoder(const fly_dense &d, const void *x, bool x_f16, int64_t ldx, int
              EncoderEpilogue{d.enc_b.p, gain, u, u16, ldu}, d.gemm_tile, 1, st);
 }
 
+// ws: `room` bytes, at least those of one part; a smaller room than head_ws takes fewer parts.
 template <typename S>
 void run_head(const fly_dense &d, const S *state, int64_t lds, const int32_t *src, const float *cbase, int64_t batch,
-              float *logits, float *wdl, void *ws, hipStream_t st) {
+              float *logits, float *wdl, void *ws, size_t room, hipStream_t st) {
   LaunchTimer timer(FLY_K_HEAD, st);
   char *base = static_cast<char *>(ws);
   _Float16 *rh = reinterpret_cast<_Float16 *>(base);
@@ -579,7 +589,8 @@ void run_head(const fly_dense &d, const S *state, int64_t lds, const int32_t *sr
                      d.eps, d.clip, d.n_out, batch, rh, rl, d.kp_head);
   check_launch("normalised outputs");
   const int64_t ldc = head_ld(d);
-  const int splits = head_splits(d, batch);
+  int splits = head_splits(d, batch);
+  while (splits > 1 && head_ws_rows(d, batch, splits * batch) > room) --splits;
   gemm_split(Split{d.head_hi.p, d.head_lo.p, d.head_rows(), nullptr}, Split{rh, rl, batch, nullptr}, d.kp_head,
              d.head_unscale, HeadEpilogue{ct, ldc, batch * ldc}, d.gemm_tile, splits, st);
   const bool avec = d.n_moves % 4 == 0 && ldc % 4 == 0 && aligned(logits, 16);
@@ -713,7 +724,7 @@ extern "C" int fly_head(const fly_dense *d, const float *r, int64_t ldr, int64_t
     if (!batch) return;
     FLY_REQUIRE(r && ldr >= batch && logits && wdl, "bad argument");
     FLY_REQUIRE(ws && ws_bytes >= head_ws(*d, batch) && aligned(ws, 256), "workspace too small or misaligned");
-    run_head<float>(*d, r, ldr, nullptr, nullptr, batch, logits, wdl, ws, as_stream(stream));
+    run_head<float>(*d, r, ldr, nullptr, nullptr, batch, logits, wdl, ws, ws_bytes, as_stream(stream));
   });
 }
 
@@ -722,11 +733,11 @@ namespace {
 
 // Scratch of one block of `blk` boards of the model forward: the encoder's output u (float32, padded rows), the
 // two state buffers, then the encoder's operand split or the head's (they never live at once).
-size_t model_ws_block(const fly_plan &plan, const fly_dense &d, int64_t blk) {
+size_t model_ws_block(const fly_plan &plan, const fly_dense &d, int64_t blk, size_t head_bytes) {
   const size_t es = plan.mode == FLY_MODE_DEVIATION_F16 ? sizeof(_Float16) : sizeof(float);
   return align256((size_t)plan.n_in * state_ld(blk, sizeof(float)) * sizeof(float)) +
          align256(2 * (size_t)plan.max_rows * (size_t)state_ld(blk, es) * es + 256) + plan_pieces_bytes(plan, blk) +
-         std::max(encoder_ws(d, blk), head_ws(d, blk));
+         std::max(encoder_ws(d, blk), head_bytes);
 }
 
 void check_model_args(const fly_plan *plan, const fly_dense *d, const void *x, int64_t ldx, int64_t batch,
@@ -739,10 +750,11 @@ void check_model_args(const fly_plan *plan, const fly_dense *d, const void *x, i
   if (batch) FLY_REQUIRE(x && ldx >= d->k && logits && wdl, "bad argument");
 }
 
-// The forward in blocks of at most `blk` boards, each using the scratch at ws (model_ws_block(blk) bytes).
+// The forward in blocks of at most `blk` boards, each using the ws_bytes of scratch at ws (at least model_ws_block with
+// one part of the head).
 void model_forward_blocks(const fly_plan &plan, const fly_dense &d, const void *x, bool x_f16, int64_t ldx,
-                          int64_t batch, float input_gain, float *logits, float *wdl, void *ws, int64_t blk,
-                          hipStream_t st) {
+                          int64_t batch, float input_gain, float *logits, float *wdl, void *ws, size_t ws_bytes,
+                          int64_t blk, hipStream_t st) {
   char *base = static_cast<char *>(ws);
   float *u = reinterpret_cast<float *>(base);
   base += align256((size_t)plan.n_in * state_ld(blk, sizeof(float)) * sizeof(float));
@@ -752,6 +764,7 @@ void model_forward_blocks(const fly_plan &plan, const fly_dense &d, const void *
   float *pieces = reinterpret_cast<float *>(base);   // the sums of split rows' pieces
   base += plan_pieces_bytes(plan, blk);
   void *scratch_ops = base;  // the encoder's operand split, then the head's
+  const size_t room = ws_bytes - (size_t)(base - static_cast<char *>(ws));
   const size_t xelem = x_f16 ? sizeof(_Float16) : sizeof(float);
   for (int64_t c0 = 0; c0 < batch; c0 += blk) {
     const int64_t nb = std::min(blk, batch - c0);
@@ -763,10 +776,10 @@ void model_forward_blocks(const fly_plan &plan, const fly_dense &d, const void *
     run_encoder(d, xb, x_f16, ldx, nb, input_gain, u, nullptr, ldu, scratch_ops, st);
     if (plan.mode == FLY_MODE_DEVIATION_F16) {
       const _Float16 *fin = run_cone_steps<_Float16, float>(plan, u, ldu, nb, true, states, pieces, st);
-      run_head<_Float16>(d, fin, lds, plan.out_src.p, plan.cbase.p, nb, lb, wb, scratch_ops, st);
+      run_head<_Float16>(d, fin, lds, plan.out_src.p, plan.cbase.p, nb, lb, wb, scratch_ops, room, st);
     } else {
       const float *fin = run_cone_steps<float, float>(plan, u, ldu, nb, true, states, pieces, st);
-      run_head<float>(d, fin, lds, plan.out_src.p, plan.cbase.p, nb, lb, wb, scratch_ops, st);
+      run_head<float>(d, fin, lds, plan.out_src.p, plan.cbase.p, nb, lb, wb, scratch_ops, room, st);
     }
   }
 }
@@ -802,12 +815,16 @@ void *static_scratch() {
 }
 
 // Boards per block that fit the static scratch: the whole batch if it fits, else the largest multiple of 64
-// that does; 0 when not even min(batch, 64) boards fit.
+// that does; 0 when not even min(batch, 64) boards fit.  Counted with one part of the head: its further parts take what
+// is left of the array.
+size_t static_need(const fly_plan &plan, const fly_dense &d, int64_t blk) {
+  return model_ws_block(plan, d, blk, head_ws_rows(d, blk, blk));
+}
 int64_t static_block(const fly_plan &plan, const fly_dense &d, int64_t batch) {
   const size_t cap = FLY_STATIC_SCRATCH_BYTES;
-  if (model_ws_block(plan, d, batch) <= cap) return batch;
+  if (static_need(plan, d, batch) <= cap) return batch;
   for (int64_t b = (batch - 1) / 64 * 64; b >= 64; b -= 64)
-    if (model_ws_block(plan, d, b) <= cap) return b;
+    if (static_need(plan, d, b) <= cap) return b;
   return 0;
 }
 
@@ -822,19 +839,21 @@ extern "C" int fly_model_forward_static(const fly_plan *plan, const fly_dense *d
     if (!batch) return;
     const int64_t blk = static_block(*plan, *d, batch);
     FLY_REQUIRE(blk > 0, "fly_model_forward_static: one block of " + std::to_string(std::min<int64_t>(batch, 64)) +
-                             " boards needs " + std::to_string(model_ws_block(*plan, *d, std::min<int64_t>(batch, 64))) +
+                             " boards needs " + std::to_string(static_need(*plan, *d, std::min<int64_t>(batch, 64))) +
                              " bytes of scratch, above the static array's " +
                              std::to_string((size_t)FLY_STATIC_SCRATCH_BYTES) + " (use fly_model_forward)");
     void *ws = static_scratch();
     NoLaunchEvents quiet;   // the profiler's launch events would be created here: this entry point creates nothing
-    model_forward_blocks(*plan, *d, x, x_f16 != 0, ldx, batch, input_gain, logits, wdl, ws, blk, as_stream(stream));
+    model_forward_blocks(*plan, *d, x, x_f16 != 0, ldx, batch, input_gain, logits, wdl, ws, FLY_STATIC_SCRATCH_BYTES, blk,
+                         as_stream(stream));
   });
 }
 
 extern "C" size_t fly_model_workspace(const fly_plan *plan, const fly_dense *d, int64_t batch) {
   if (!plan || !d) return 0;
   // boards per block: the whole batch while the state stays below 2 GiB (io_block)
-  return model_ws_block(*plan, *d, io_block(*plan, batch));
+  const int64_t blk = io_block(*plan, batch);
+  return model_ws_block(*plan, *d, blk, head_ws(*d, blk));
 }
 
 extern "C" int fly_model_forward(const fly_plan *plan, const fly_dense *d, const void *x, int32_t x_f16, int64_t ldx,
@@ -846,7 +865,7 @@ extern "C" int fly_model_forward(const fly_plan *plan, const fly_dense *d, const
     FLY_REQUIRE(ws && ws_bytes >= fly_model_workspace(plan, d, batch), "workspace too small");
     FLY_REQUIRE(aligned(ws, 256), "workspace must be 256-byte aligned");
     // Boards run in blocks whose state stays below 2 GiB (one block below about 6,400 boards in float16).
-    model_forward_blocks(*plan, *d, x, x_f16 != 0, ldx, batch, input_gain, logits, wdl, ws, io_block(*plan, batch),
-                         as_stream(stream));
+    model_forward_blocks(*plan, *d, x, x_f16 != 0, ldx, batch, input_gain, logits, wdl, ws, ws_bytes,
+                         io_block(*plan, batch), as_stream(stream));
   });
 }

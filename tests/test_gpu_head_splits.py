@@ -51,3 +51,25 @@ def test_head_in_parts_matches_float64(n_out, n_moves, batch):
         # 22-bit operands and float32 sums of at most 3 (n_out + 1) products of order 1 / sqrt(n_out): 1e-5 of the scale
         for got, ref in ((logits, want), (wdl, f64["value"])):
             assert float((got.double() - ref).abs().max()) < 1e-5 * max(1.0, float(ref.abs().max())), splits
+
+
+def test_workspace_of_a_batch_holds_every_smaller_one():
+    """A smaller batch may run in more parts than a larger one (576 boards of the full-size head in two, 640 in one): the
+    last block of a forward and a caller who keeps one workspace both use a larger batch's workspace for it."""
+    from chessfly import _hip
+    lib = _hip.load()
+    n_out, n_moves = 100, 4168
+    z = lambda *shape: torch.zeros(shape, device=DEV)
+    maps = [z(n_moves, n_out), z(n_moves), z(64, n_out), z(64), z(64, n_out), z(64), z(3, n_out), z(3)]
+    squares = torch.zeros(n_moves, dtype=torch.int32, device=DEV)
+    mean, var, enc_w, enc_b = z(n_out), z(n_out) + 1, z(5, 7), z(5)
+    desc = _hip.HeadDesc(n_out, n_moves, mean.data_ptr(), var.data_ptr(), 1e-8, 8.0, *[p.data_ptr() for p in maps],
+                         squares.data_ptr(), squares.data_ptr())
+    handle = ctypes.c_void_p()
+    _hip.check(lib.fly_dense_create(ctypes.byref(desc), enc_w.data_ptr(), 7, 7, enc_b.data_ptr(), 5,
+                                    _hip.stream(mean.device), ctypes.byref(handle)), "fly_dense_create")
+    dense = _hip.Handle(handle, "fly_dense_destroy")
+    sizes = [int(lib.fly_head_workspace(dense.handle, b)) for b in range(1, 3000)]
+    assert all(a <= b for a, b in zip(sizes, sizes[1:]))
+    # room for two parts of 576 boards beside the operands (2 x 2 bytes, 128 columns): float32 rows of 4,299 values
+    assert sizes[639] >= 2 * 576 * 4299 * 4
