@@ -479,9 +479,11 @@ __global__ void k_sweep_ranges(const int32_t *__restrict__ off, int K, int64_t n
   }
 }
 
-// The staged step's tables of t's structure: none where its columns are out of order.
+// The staged step's tables of t's structure: none where its columns are out of order, or where a forced sweep's matrix is
+// so small that its bands' sums outgrow their place behind the state rows or a band holds no whole 16-byte piece.
 template <typename C>
 void build_stage(const int32_t *rowptr, const C *cols, SweepTables &t, hipStream_t st) {
+  if (t.nrows < 64 || t.ncols < 64) return;
   DevArray<int32_t> bad(1);
   const int32_t zero = 0;
   FLY_HIP(hipMemcpyAsync(bad.p, &zero, sizeof(zero), hipMemcpyHostToDevice, st));
