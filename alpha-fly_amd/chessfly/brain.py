@@ -49,14 +49,17 @@ def _transpose_order(rows: torch.Tensor, cols: torch.Tensor, n_rows: int) -> tor
 
 
 def _spmm(crow32, col32, val, n_rows: int, n_cols: int, x: torch.Tensor, out: torch.Tensor | None = None,
-          val_ids32: torch.Tensor | None = None) -> torch.Tensor:
+          val_ids32: torch.Tensor | None = None, used: int | None = None) -> torch.Tensor:
     """y (n_rows, B) = A x on the device (fly_spmm); x (n_cols, B) float32.  With `out`, y is added to it; with
-    `val_ids32` the values are val[val_ids32[e]]."""
+    `val_ids32` the values are val[val_ids32[e]]; with `used` only the first columns are computed and the others 0."""
     x = x.contiguous()
     batch = x.shape[1]
     y = torch.empty(n_rows, batch, dtype=torch.float32, device=x.device) if out is None else out
+    cols = batch if used is None else used
+    if cols < batch:
+        y[:, cols:] = 0.0
     _hip.check(_hip.load().fly_spmm(crow32.data_ptr(), col32.data_ptr(), val.data_ptr(), _hip.ptr(val_ids32),
-                                    val.numel(), n_rows, n_cols, x.data_ptr(), max(batch, 1), batch, y.data_ptr(),
+                                    val.numel(), n_rows, n_cols, x.data_ptr(), max(batch, 1), cols, y.data_ptr(),
                                     max(batch, 1), int(out is not None), _hip.stream(x.device)), "fly_spmm")
     return y
 
@@ -279,7 +282,10 @@ class _ConeRecurrence(torch.autograd.Function):
             k, pdef, alpha = flat[3 * (t - 1):3 * t]
             rows, op = cone.row_counts[t], cone.ops[t]
             prev32, usrc32 = cone.step_tables32(t)
-            if op is not None:
+            if op is not None and pad:          # sums in fly_spmm's 8 groups, as one column per lane has them
+                crow32, col32, n_rows, n_cols = op._structure()
+                y = _spmm(crow32, col32, _gathered(op, w, False), n_rows, n_cols, h, used=given)
+            elif op is not None:
                 y = _product(op, w, h)
             else:
                 y = torch.empty(rows, batch, dtype=torch.float32, device=dev)

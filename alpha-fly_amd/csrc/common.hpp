@@ -74,7 +74,7 @@ inline int current_device() {
 //
 // A block is handed on only once no GPU work can still use it: alloc() waits for the device if the block came back
 // after the last such wait, unless a QuietRelease said then that its work was over.  Releasing makes no GPU call while
-// the block stays here, so an object may go away while a stream is being captured.  Safe to use from several threads.
+// the block stays here (a wait there would spoil a stream capture, as hipFree does).  Safe to use from several threads.
 class DevicePool {
  public:
   static DevicePool &get() {

@@ -1082,7 +1082,9 @@ extern "C" int fly_spmm(const int32_t *rowptr, const int32_t *col, const float *
       hipLaunchKernelGGL(k_spmv, dim3(blocks_for(nrows, 16)), dim3(256), 0, as_stream(stream), b);
     } else if (batch >= 4 && vec4_ok(x, ldx) && vec4_ok(y, ldy)) {
       const int tg = tuning_snapshot().spmm_groups;
-      const int g = tg == 2 || tg == 8 ? tg : 4;
+      // 8 groups where the batch is ragged (a leading dimension of whole 16-byte pieces behind it): a row's sum then
+      // has the bits that one column per lane gives it, 8 shares of its non-zeros added in a tree
+      const int g = tg == 2 || tg == 4 || tg == 8 ? tg : (batch % 4 ? 8 : 4);
       const int width = 64 / g * 4;   // columns per chunk
       a.chunks = (int32_t)((batch + width - 1) / width);
       if (g == 2)

@@ -744,3 +744,22 @@ def test_cone_gradients_of_ragged_batches_match_the_oracle(batch, swept):
     for g, r, name in zip(got, want, ("out", "u_in", "log_gain", "bias", "alpha_logit")):
         assert g.shape == r.shape, name
         _close(g, r, 1e-4, f"ragged B={batch} swept={swept} {name}")
+
+
+@pytest.mark.parametrize("batch", [1, 2, 3, 5, 31, 33, 67])
+def test_padded_product_has_the_unpadded_products_bits(batch):
+    """fly_spmm over a ragged batch whose rows are padded to 16 bytes (16-byte lanes) sums in the same order as over rows
+    of the batch alone (one column per lane), and the columns behind the batch are 0."""
+    from chessfly.brain import _spmm
+    g = torch.Generator().manual_seed(batch)
+    rows, cols = 300, 500
+    per = torch.randint(0, 90, (rows,), generator=g)
+    per[0], per[1] = 0, 400
+    crow = torch.cat((torch.zeros(1, dtype=torch.int64), per.cumsum(0))).to(torch.int32).to(DEV)
+    col = torch.randint(0, cols, (int(per.sum()),), generator=g).to(torch.int32).to(DEV)
+    val = torch.randn(int(per.sum()), generator=g).to(DEV)
+    x = torch.randn(cols, batch, generator=g).to(DEV)
+    padded = torch.nn.functional.pad(x, (0, -batch % 4), value=float("nan"))
+    want = _spmm(crow, col, val, rows, cols, x)
+    got = _spmm(crow, col, val, rows, cols, padded, used=batch)
+    assert torch.equal(got[:, :batch], want) and bool((got[:, batch:] == 0).all())
