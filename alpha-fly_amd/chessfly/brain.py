@@ -247,6 +247,20 @@ def _product(op, w: torch.Tensor, x: torch.Tensor, transposed: bool = False, out
     return _spmm(crow32, col32, _gathered(op, w, transposed), n_rows, n_cols, x, out=out)
 
 
+def _pad_columns(batch: int, rows: int) -> int:
+    """Columns of zeros behind a batch of the training recurrence, whose states have up to `rows` rows.  Rows of whole
+    128-byte lines (32 columns) from 25 positions on: the products gather pieces of 32 columns, which otherwise straddle
+    two lines (full-size network, ms per forward and backward with rows of whole 16 bytes and of whole lines: 27
+    positions 4.73 / 4.45, 36 5.08 / 4.97, 67 7.40 / 5.93, 68 6.29 / 5.45, 100 7.51 / 6.18, 145 10.99 / 7.88, 200
+    11.27 / 8.71).  Below that rows of whole 16 bytes, since wider ones gain nothing (12 positions 4.15 / 4.33, 20 4.28 /
+    4.31).  A state that would pass 2 GiB is padded less, or not at all."""
+    for unit in (32, 4) if batch > 24 else (4,):
+        pad = -batch % unit
+        if rows * (batch + pad) * 4 < 2 ** 31:
+            return pad
+    return 0
+
+
 class _ConeRecurrence(torch.autograd.Function):
     """Steps 1..T of the light cone under autograd, float32 (brain.py:313-327): per step the sub-matrix
     product on the device (its values read from the whole edge-weight vector w at the sub-matrix's edge ids),
@@ -257,11 +271,12 @@ class _ConeRecurrence(torch.autograd.Function):
     dL/dw (chunk-major above 64 columns, so the gathers share one chunk of grad_y in the caches).  The transposed
     passes work in the transposed order of the whole weight vector (rnn's W^T), where every step's ids rise along
     the pass: they read A_t^T's values from w in that order and add into dL/dw kept in that order, which one gather
-    at the end puts back in the weight vector's order.  Batches that are not a multiple of 4 run with up to 3 columns
-    of zeros behind them (zero drive, zero state kept, zero gradient), so every row starts on 16 bytes and the same
-    products serve them: through fly_spmm and fly_sddmm, which then take one column per lane, a training step of 67
-    positions on the full-size network took 14.9 ms, padded 6.3 ms (256 positions: 9.4 ms).  Only a batch whose padded
-    state would pass 2 GiB stays as it is.  Inputs after u_in and w, per step t: k_t, the previous resting state
+    at the end puts back in the weight vector's order.  Batches run with columns of zeros behind them where their
+    rows do not start on 16 bytes or on a line (_pad_columns: zero drive, zero state kept, zero gradient), so the
+    same products serve them.  The forward products of a ragged batch (not a multiple of 4) go through fly_spmm, whose order of a row's sum is
+    the same on 16-byte lanes as on one column per lane; a swept product's state is further from float64 (7.0e-8 against
+    6.0e-8), which costs a gradient more where a drive lies at a clamp's bound.  67 positions: 14.9 ms through products of
+    one column per lane, 5.9 padded.  Inputs after u_in and w, per step t: k_t, the previous resting state
     c_{t-1}[R_t] and alpha[R_t] (each (|R_t|, 1)).  Returns h_T, (|R_T|, B)."""
 
     @staticmethod
@@ -270,9 +285,7 @@ class _ConeRecurrence(torch.autograd.Function):
         dev = u_in.device
         st = _hip.stream(dev)
         given = u_in.shape[1]
-        pad = -given % 4
-        if max(cone.row_counts) * (given + pad) * 4 >= 2 ** 31:
-            pad = 0
+        pad = _pad_columns(given, max(cone.row_counts))
         u_in = nn.functional.pad(u_in, (0, pad)) if pad else u_in.contiguous()
         batch = given + pad
         ld = max(batch, 1)
@@ -282,11 +295,13 @@ class _ConeRecurrence(torch.autograd.Function):
             k, pdef, alpha = flat[3 * (t - 1):3 * t]
             rows, op = cone.row_counts[t], cone.ops[t]
             prev32, usrc32 = cone.step_tables32(t)
-            if op is not None and pad:          # sums in fly_spmm's 8 groups, as one column per lane has them
+            if op is not None and pad and given % 4:   # sums in fly_spmm's 8 groups, as one column per lane has them
                 crow32, col32, n_rows, n_cols = op._structure()
                 y = _spmm(crow32, col32, _gathered(op, w, False), n_rows, n_cols, h, used=given)
             elif op is not None:
                 y = _product(op, w, h)
+                if pad:
+                    y[:, given:] = 0.0          # an infinite weight makes NaN of a column of zeros
             else:
                 y = torch.empty(rows, batch, dtype=torch.float32, device=dev)
             hn = torch.empty(rows, batch, dtype=torch.float32, device=dev)

@@ -710,10 +710,10 @@ def test_full_scale_train_step_gradients_match_the_oracle(full_net, batch):
         _close(got[name], want[name], 1e-3, name)
 
 
-@pytest.mark.parametrize("batch", [1, 3, 66, 201])
+@pytest.mark.parametrize("batch", [1, 3, 25, 36, 66, 201])
 @pytest.mark.parametrize("swept", [False, True])
 def test_cone_gradients_of_ragged_batches_match_the_oracle(batch, swept):
-    """forward_io under autograd at batches that are not a multiple of 4, which run with columns of zeros behind them:
+    """forward_io under autograd at batches that are no multiple of 4 or of 32, which run with columns of zeros behind them:
     outputs and gradients against the oracle in float64, in one chunk and with a ragged last one, and with the sweep
     forced; the gradient of u_in has the batch's own shape."""
     from chessfly import _hip
@@ -763,3 +763,31 @@ def test_padded_product_has_the_unpadded_products_bits(batch):
     want = _spmm(crow, col, val, rows, cols, x)
     got = _spmm(crow, col, val, rows, cols, padded, used=batch)
     assert torch.equal(got[:, :batch], want) and bool((got[:, batch:] == 0).all())
+
+
+@pytest.mark.parametrize("batch", [36, 37])
+def test_an_infinite_weight_gives_a_padded_batch_no_nan_of_its_own(batch):
+    """A weight that overflows drives its neuron to the clamp's bound at every position of a batch without zeros in the
+    state: outputs stay finite, and so do alpha's gradients there, with columns of zeros behind the batch."""
+    from chessfly.synthetic import GraphSpec, synthetic_connectome
+    conn = synthetic_connectome(GraphSpec(n=400, edges=4000, n_sensory=100, n_output=50, seed=5))
+    rnn, _ = _rnn_pair(conn, 3)
+    post = int(conn.post[conn.post >= 350][0])
+    edge = int(((conn.post == post) & (conn.sign > 0)).nonzero()[0])
+    with torch.no_grad():
+        rnn.bias.fill_(0.5)                     # every state above 0, at rest and under the drive
+        rnn.log_gain.fill_(-20.0)
+        rnn.log_gain[edge] = 200.0              # exp overflows
+    g = torch.Generator().manual_seed(1)
+    u = torch.rand(100, batch, generator=g).to(DEV).requires_grad_(True)
+    out = rnn.forward_io(u, torch.arange(0, 100, device=DEV), torch.arange(350, 400, device=DEV), 3)
+    plain = [rnn.forward_io(u[:, i:i + 4], torch.arange(0, 100, device=DEV), torch.arange(350, 400, device=DEV), 3)
+             for i in (0, batch - 4)]
+    assert torch.equal(out.isfinite()[:, :4], plain[0].isfinite())
+    assert torch.equal(out.isfinite()[:, -4:], plain[1].isfinite())
+    out.sum().backward()
+    got = rnn.alpha_logit.grad.clone()
+    rnn.alpha_logit.grad = None
+    sum(rnn.forward_io(u[:, i:i + 4], torch.arange(0, 100, device=DEV), torch.arange(350, 400, device=DEV), 3).sum()
+        for i in range(0, 36, 4)).backward()
+    assert torch.equal(got.isfinite(), rnn.alpha_logit.grad.isfinite())
