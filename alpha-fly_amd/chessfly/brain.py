@@ -49,14 +49,15 @@ def _transpose_order(rows: torch.Tensor, cols: torch.Tensor, n_rows: int) -> tor
 
 
 def _spmm(crow32, col32, val, n_rows: int, n_cols: int, x: torch.Tensor, out: torch.Tensor | None = None,
-          val_ids32: torch.Tensor | None = None, used: int | None = None) -> torch.Tensor:
+          val_ids32: torch.Tensor | None = None, used: int | None = None, clear: bool = True) -> torch.Tensor:
     """y (n_rows, B) = A x on the device (fly_spmm); x (n_cols, B) float32.  With `out`, y is added to it; with
-    `val_ids32` the values are val[val_ids32[e]]; with `used` only the first columns are computed and the others 0."""
+    `val_ids32` the values are val[val_ids32[e]]; with `used` only the first columns are computed and the others 0,
+    or left as they are without `clear`."""
     x = x.contiguous()
     batch = x.shape[1]
     y = torch.empty(n_rows, batch, dtype=torch.float32, device=x.device) if out is None else out
     cols = batch if used is None else used
-    if cols < batch:
+    if cols < batch and clear:
         y[:, cols:] = 0.0
     _hip.check(_hip.load().fly_spmm(crow32.data_ptr(), col32.data_ptr(), val.data_ptr(), _hip.ptr(val_ids32),
                                     val.numel(), n_rows, n_cols, x.data_ptr(), max(batch, 1), cols, y.data_ptr(),
@@ -76,17 +77,20 @@ def _sweep_tables(holder, crow32, col32, n_rows: int, n_cols: int, attr: str = "
     return tables
 
 
-def _spmm_swept(col32, val, tables, n_rows: int, x: torch.Tensor, records: torch.Tensor | None = None) -> torch.Tensor:
+def _spmm_swept(col32, val, tables, n_rows: int, x: torch.Tensor, records: torch.Tensor | None = None,
+                used: int | None = None) -> torch.Tensor:
     """y (n_rows, B) = A x as a banded sweep (fly_spmm_swept) from {column, weight} records (`records`, or built from
-    col32 and val); x (n_cols, B) float32, contiguous and 16-byte aligned, with B a multiple of 4."""
-    batch = x.shape[1]
-    y = torch.empty(n_rows, batch, dtype=torch.float32, device=x.device)
+    col32 and val); x (n_cols, B) float32, contiguous and 16-byte aligned, with B a multiple of 4.  With `used`, a
+    multiple of 4 too, only the first columns are computed and the others left as they are."""
+    ld = x.shape[1]
+    batch = ld if used is None else used
+    y = torch.empty(n_rows, ld, dtype=torch.float32, device=x.device)
     if records is None:
         records = torch.stack((col32, val.contiguous().view(torch.int32)), dim=1)
     lib = _hip.load()
     ws = _hip.workspace(lib.fly_spmm_swept_workspace(tables.handle, batch), x.device)
-    _hip.check(lib.fly_spmm_swept(tables.handle, records.data_ptr(), col32.numel(), x.data_ptr(), batch, batch,
-                                  y.data_ptr(), batch, ws.data_ptr(), ws.numel(), _hip.stream(x.device)),
+    _hip.check(lib.fly_spmm_swept(tables.handle, records.data_ptr(), col32.numel(), x.data_ptr(), ld, batch,
+                                  y.data_ptr(), ld, ws.data_ptr(), ws.numel(), _hip.stream(x.device)),
                "fly_spmm_swept")
     return y
 
@@ -226,8 +230,10 @@ def backward_work(t_crow: torch.Tensor, seg: int = 256):
     return items, splits, int(extra.sum())
 
 
-def _product(op, w: torch.Tensor, x: torch.Tensor, transposed: bool = False, out: torch.Tensor | None = None):
-    """A x (or A^T x) with A's values from w, gathered once per weight tensor into the structure's order.
+def _product(op, w: torch.Tensor, x: torch.Tensor, transposed: bool = False, out: torch.Tensor | None = None,
+             used: int | None = None):
+    """A x (or A^T x) with A's values from w, gathered once per weight tensor into the structure's order.  With `used`
+    (A x only) just the first columns are computed and the others left as they are.
     Every product of a training step over one structure shares the gathered copy, so each reads its values as
     a stream; reading w through value ids instead would cost a random line per non-zero in the transposed
     order, on every call."""
@@ -238,17 +244,17 @@ def _product(op, w: torch.Tensor, x: torch.Tensor, transposed: bool = False, out
             return _spmv_work(crow32, col32, _gathered(op, w, True), n_rows, n_cols, x, op._backward_work(), out=out)
     else:
         crow32, col32, n_rows, n_cols = op._structure()
-        batch = x.shape[1]
+        batch = x.shape[1] if used is None else used
         if out is None and x.dtype == torch.float32 and batch >= 4 and batch % 4 == 0:
             tables = _sweep_tables(op, crow32, col32, n_rows, n_cols)
             x = x.contiguous()
             if tables is not None and x.data_ptr() % 16 == 0:
-                return _spmm_swept(col32, None, tables, n_rows, x, records=_records(op, w, False))
-    return _spmm(crow32, col32, _gathered(op, w, transposed), n_rows, n_cols, x, out=out)
+                return _spmm_swept(col32, None, tables, n_rows, x, records=_records(op, w, False), used=used)
+    return _spmm(crow32, col32, _gathered(op, w, transposed), n_rows, n_cols, x, out=out, used=used, clear=False)
 
 
 def _pad_columns(batch: int, rows: int) -> int:
-    """Columns of zeros behind a batch of the training recurrence, whose states have up to `rows` rows.  Rows of whole
+    """Columns kept free behind a batch of the training recurrence, whose states have up to `rows` rows.  Rows of whole
     128-byte lines (32 columns) from 25 positions on: the products gather pieces of 32 columns, which otherwise straddle
     two lines (full-size network, ms per forward and backward with rows of whole 16 bytes and of whole lines: 27
     positions 4.73 / 4.45, 36 5.08 / 4.97, 67 7.40 / 5.93, 68 6.29 / 5.45, 100 7.51 / 6.18, 145 10.99 / 7.88, 200
@@ -271,57 +277,62 @@ class _ConeRecurrence(torch.autograd.Function):
     dL/dw (chunk-major above 64 columns, so the gathers share one chunk of grad_y in the caches).  The transposed
     passes work in the transposed order of the whole weight vector (rnn's W^T), where every step's ids rise along
     the pass: they read A_t^T's values from w in that order and add into dL/dw kept in that order, which one gather
-    at the end puts back in the weight vector's order.  Batches run with columns of zeros behind them where their
-    rows do not start on 16 bytes or on a line (_pad_columns: zero drive, zero state kept, zero gradient), so the
-    same products serve them.  The forward products of a ragged batch (not a multiple of 4) go through fly_spmm, whose order of a row's sum is
-    the same on 16-byte lanes as on one column per lane; a swept product's state is further from float64 (7.0e-8 against
-    6.0e-8), which costs a gradient more where a drive lies at a clamp's bound.  67 positions: 14.9 ms through products of
-    one column per lane, 5.9 padded.  Inputs after u_in and w, per step t: k_t, the previous resting state
-    c_{t-1}[R_t] and alpha[R_t] (each (|R_t|, 1)).  Returns h_T, (|R_T|, B)."""
+    at the end puts back in the weight vector's order.  States, drives and their gradients have rows of whole 16 bytes
+    or whole lines (_pad_columns), which serve every batch with the same products; only the batch's own columns are
+    computed.  Behind a ragged batch (not a multiple of 4) up to 3 columns of zeros make the columns of the products
+    over A^T a multiple of 4: each of the two buffers that holds them is cleared in one launch, since a small network's
+    step is bound by its launches (3,000 neurons, 36 positions: 1.15 ms with the columns behind the batch computed or
+    cleared step by step, 1.03 without).  The forward products of a ragged batch go through fly_spmm, whose order of a
+    row's sum is the same on 16-byte lanes as on one column per lane; a swept product's state is further from float64
+    (7.0e-8 against 6.0e-8), which costs a gradient more where a drive lies at a clamp's bound.  67 positions: 14.9 ms
+    through products of one column per lane, 5.9 on such rows.  Inputs after u_in and w, per step t: k_t, the previous
+    resting state c_{t-1}[R_t] and alpha[R_t] (each (|R_t|, 1)).  Returns h_T, (|R_T|, B)."""
 
     @staticmethod
     def forward(ctx, cone, h_max, rnn, u_in, w, *flat):
         lib = _hip.load()
         dev = u_in.device
         st = _hip.stream(dev)
-        given = u_in.shape[1]
-        pad = _pad_columns(given, max(cone.row_counts))
-        u_in = nn.functional.pad(u_in, (0, pad)) if pad else u_in.contiguous()
-        batch = given + pad
-        ld = max(batch, 1)
+        u_in = u_in.contiguous()
+        batch = u_in.shape[1]
+        pad = _pad_columns(batch, max(cone.row_counts))
+        ld, ldu = max(batch + pad, 1), max(batch, 1)
+        zeros = -batch % 4 if pad else 0
         hs, ys = [], []
+        # The last state is the result, in rows of the batch alone.  The earlier ones are read by a later step: those of a
+        # ragged batch share a buffer, whose columns of zeros are cleared once.
+        state = None
+        if zeros:
+            state = torch.empty(sum(cone.row_counts[1:cone.steps]), ld, dtype=torch.float32, device=dev)
+            state[:, batch:batch + zeros].zero_()
+            state = state.split(cone.row_counts[1:cone.steps])
         h = None
         for t in range(1, cone.steps + 1):
             k, pdef, alpha = flat[3 * (t - 1):3 * t]
             rows, op = cone.row_counts[t], cone.ops[t]
             prev32, usrc32 = cone.step_tables32(t)
-            if op is not None and pad and given % 4:   # sums in fly_spmm's 8 groups, as one column per lane has them
-                crow32, col32, n_rows, n_cols = op._structure()
-                y = _spmm(crow32, col32, _gathered(op, w, False), n_rows, n_cols, h, used=given)
-            elif op is not None:
-                y = _product(op, w, h)
-                if pad:
-                    y[:, given:] = 0.0          # an infinite weight makes NaN of a column of zeros
+            last = t == cone.steps
+            if op is not None:
+                y = _product(op, w, h, used=batch)
             else:
-                y = torch.empty(rows, batch, dtype=torch.float32, device=dev)
-            hn = torch.empty(rows, batch, dtype=torch.float32, device=dev)
+                y = torch.empty(rows, ld, dtype=torch.float32, device=dev)
+            hn = torch.empty(rows, batch if last else ld, dtype=torch.float32, device=dev) \
+                if last or state is None else state[t - 1]
             # operands bound to names: a temporary freed inside the argument list could be reused (and
             # overwritten on the stream) by the next one before the kernel reads it
             k, pdef, alpha = k.contiguous(), pdef.contiguous(), alpha.contiguous()
             _hip.check(lib.fly_train_step_forward(
                 rows, batch, y.data_ptr(), ld, int(op is not None), k.data_ptr(),
                 pdef.data_ptr(), alpha.data_ptr(),
-                _hip.ptr(prev32 if h is not None and h.shape[0] else None), usrc32.data_ptr(), u_in.data_ptr(), ld,
-                _hip.ptr(h), ld, float(h_max), hn.data_ptr(), ld, st), "fly_train_step_forward")
-            if pad:
-                hn[:, given:] = 0.0         # a column of no position adds nothing to a gradient
+                _hip.ptr(prev32 if h is not None and h.shape[0] else None), usrc32.data_ptr(), u_in.data_ptr(), ldu,
+                _hip.ptr(h), ld, float(h_max), hn.data_ptr(), ldu if last else ld, st), "fly_train_step_forward")
             hs.append(hn)
             ys.append(y)
             h = hn
         ctx.cone, ctx.h_max, ctx.rnn = cone, float(h_max), rnn
-        ctx.given = given
+        ctx.ld, ctx.zeros = ld, zeros
         ctx.save_for_backward(u_in, w, *hs, *ys, *flat)
-        return h[:, :given].contiguous() if pad else h
+        return h
 
     @staticmethod
     def backward(ctx, grad_h):
@@ -334,9 +345,13 @@ class _ConeRecurrence(torch.autograd.Function):
         dev = u_in.device
         st = _hip.stream(dev)
         batch = u_in.shape[1]
-        pad = batch - ctx.given
-        ld = max(batch, 1)
-        g = nn.functional.pad(grad_h, (0, pad)) if pad else grad_h.contiguous()
+        ld, ldu = ctx.ld, max(batch, 1)
+        g, ldg = grad_h.contiguous(), ldu
+        wide = batch + ctx.zeros                      # columns of the products over A^T
+        gy_all = None
+        if ctx.zeros:                                 # one buffer for every step, its columns of zeros cleared once
+            gy_all = torch.empty(max(cone.row_counts), ld, dtype=torch.float32, device=dev)
+            gy_all[:, batch:wide].zero_()
         gu = torch.zeros_like(u_in)
         gw = torch.zeros_like(w)
         gw_t = w_pos32 = None                         # dL/dw in W^T's order, for the transposed passes
@@ -346,23 +361,23 @@ class _ConeRecurrence(torch.autograd.Function):
             rows, op = cone.row_counts[t], cone.ops[t]
             prev32, usrc32 = cone.step_tables32(t)
             h_prev = hs[t - 2] if t > 1 else None
-            gy = torch.empty(rows, batch, dtype=torch.float32, device=dev)
+            gy = torch.empty(rows, ld, dtype=torch.float32, device=dev) if gy_all is None else gy_all[:rows]
             gk = torch.empty(rows, dtype=torch.float32, device=dev)
             ga = torch.empty_like(gk)
             gpdef = torch.empty_like(gk)
-            gh_prev = torch.zeros(cone.row_counts[t - 1], batch, dtype=torch.float32, device=dev) if t > 1 else None
+            gh_prev = torch.zeros(cone.row_counts[t - 1], ld, dtype=torch.float32, device=dev) if t > 1 else None
             pdef, alpha = pdef.contiguous(), alpha.contiguous()
             _hip.check(lib.fly_train_step_backward(
-                rows, batch, g.data_ptr(), ld, ys[t - 1].data_ptr(), ld, pdef.data_ptr(),
+                rows, batch, g.data_ptr(), ldg, ys[t - 1].data_ptr(), ld, pdef.data_ptr(),
                 alpha.data_ptr(), _hip.ptr(prev32 if h_prev is not None and h_prev.shape[0] else None),
                 usrc32.data_ptr(), _hip.ptr(h_prev), ld, ctx.h_max, gy.data_ptr(), ld, gk.data_ptr(), ga.data_ptr(),
-                gpdef.data_ptr(), gu.data_ptr(), ld, _hip.ptr(gh_prev), ld, st), "fly_train_step_backward")
+                gpdef.data_ptr(), gu.data_ptr(), ldu, _hip.ptr(gh_prev), ld, st), "fly_train_step_backward")
             grads[3 * (t - 1)] = gk.view_as(k)
             grads[3 * (t - 1) + 1] = gpdef.view_as(pdef)
             grads[3 * (t - 1) + 2] = ga.view_as(alpha)
             if op is not None:
                 crow32, col32, n_rows, n_cols = op._structure()
-                if batch % 4 == 0:          # one pass over A^T: the state gradient and dL/dw together
+                if wide % 4 == 0:           # one pass over A^T: the state gradient and dL/dw together
                     t_crow32, t_col32, _ = op._transposed()
                     if w_pos32 is None:
                         w_pos32 = ctx.rnn._transposed_positions()
@@ -375,22 +390,22 @@ class _ConeRecurrence(torch.autograd.Function):
                     tables_t = _sweep_tables(op, t_crow32, t_col32, n_cols, n_rows, attr="_sweep_t")
                     if tables_t is not None:
                         records = _records(op, w, True, via=(w_t, wt_ids32))
-                        ws = _hip.workspace(lib.fly_transposed_backward_swept_workspace(tables_t.handle, batch), dev)
+                        ws = _hip.workspace(lib.fly_transposed_backward_swept_workspace(tables_t.handle, wide), dev)
                         _hip.check(lib.fly_transposed_backward_swept(
                             tables_t.handle, records.data_ptr(), t_col32.numel(), wt_ids32.data_ptr(), gy.data_ptr(),
-                            ld, h_prev.data_ptr(), ld, batch, gh_prev.data_ptr(), ld, 1, gw_t.data_ptr(), gw_t.numel(),
+                            ld, h_prev.data_ptr(), ld, wide, gh_prev.data_ptr(), ld, 1, gw_t.data_ptr(), gw_t.numel(),
                             ws.data_ptr(), ws.numel(), st), "fly_transposed_backward_swept")
                     else:
                         vals_t = _gathered(op, w, True, via=(w_t, wt_ids32))
                         items, splits, n_slots = op._backward_work()
                         partials = torch.empty(n_slots, ld, dtype=torch.float32, device=dev) if n_slots else None
                         # more than one 64-column chunk: chunk-major, each chunk's dot products kept in a workspace
-                        chunks = (batch + 63) // 64
+                        chunks = (wide + 63) // 64
                         dots = torch.empty(chunks * wt_ids32.numel(), dtype=torch.float32, device=dev) \
                             if chunks > 1 else None
                         _hip.check(lib.fly_transposed_backward(
                             t_crow32.data_ptr(), t_col32.data_ptr(), vals_t.data_ptr(), wt_ids32.data_ptr(),
-                            wt_ids32.numel(), n_cols, n_rows, gy.data_ptr(), ld, h_prev.data_ptr(), ld, batch,
+                            wt_ids32.numel(), n_cols, n_rows, gy.data_ptr(), ld, h_prev.data_ptr(), ld, wide,
                             gh_prev.data_ptr(), ld, 1, gw_t.data_ptr(), gw_t.numel(), items.data_ptr(),
                             items.shape[0], splits.data_ptr(), splits.shape[0], _hip.ptr(partials), n_slots,
                             _hip.ptr(dots), dots.numel() if dots is not None else 0, st), "fly_transposed_backward")
@@ -398,10 +413,10 @@ class _ConeRecurrence(torch.autograd.Function):
                     _product(op, w, gy, transposed=True, out=gh_prev)
                     ids32, ids = op._edge_ids()
                     _sddmm(crow32, col32, n_rows, n_cols, gy, h_prev, len(ids), out=gw, ids32=ids32)
-            g = gh_prev
+            g, ldg = gh_prev, ld
         if gw_t is not None:                          # back to the weight vector's order: gw[i] += gw_t[pos[i]]
             gw += _take(gw_t, w_pos32)
-        return (None, None, None, gu[:, :ctx.given].contiguous() if pad else gu, gw, *grads)
+        return (None, None, None, gu, gw, *grads)
 
 
 class _RestingTrajectory(torch.autograd.Function):

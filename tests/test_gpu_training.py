@@ -791,3 +791,46 @@ def test_an_infinite_weight_gives_a_padded_batch_no_nan_of_its_own(batch):
     sum(rnn.forward_io(u[:, i:i + 4], torch.arange(0, 100, device=DEV), torch.arange(350, 400, device=DEV), 3).sum()
         for i in range(0, 36, 4)).backward()
     assert torch.equal(got.isfinite(), rnn.alpha_logit.grad.isfinite())
+
+
+def test_rows_behind_a_batch_cost_no_launch_per_step():
+    """A small network's training step is bound by its launches.  A batch whose rows are widened to whole lines (36
+    positions) runs exactly the torch operations of one that fills its rows (32), and a ragged one (37) two more: the
+    columns of zeros beside its states and beside its gradients, each cleared once."""
+    from collections import Counter
+
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from chessfly.synthetic import GraphSpec, synthetic_connectome
+
+    class Count(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.ops = Counter()
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.ops[str(func)] += 1
+            return func(*args, **(kwargs or {}))
+
+    conn = synthetic_connectome(GraphSpec(n=400, edges=4000, n_sensory=100, n_output=50, seed=5))
+    rnn, _ = _rnn_pair(conn, 6)
+    ind, outd = torch.arange(0, 100, device=DEV), torch.arange(350, 400, device=DEV)
+
+    def ops(batch):
+        u = torch.randn(100, batch, device=DEV, requires_grad=True)
+        for mode in (None, Count()):                     # the first pass builds tables that the second one has
+            rnn.zero_grad(set_to_none=True)
+            with torch.autograd.set_multithreading_enabled(False):
+                if mode is None:
+                    rnn.forward_io(u, ind, outd, 6).sum().backward()
+                else:
+                    with mode:
+                        rnn.forward_io(u, ind, outd, 6).sum().backward()
+        return mode.ops
+
+    full, lines, ragged = ops(32), ops(36), ops(37)
+    assert full["aten.zeros_like.default"] >= 2          # the backward's operations are counted too
+    assert lines == full
+    free = {"aten.slice.Tensor", "aten.empty.memory_format", "aten.split_with_sizes.default"}     # no launch
+    assert {k: n for k, n in (ragged - full).items() if k not in free} == {"aten.zero_.default": 2}
+    assert not {k: n for k, n in (full - ragged).items() if k not in free}
