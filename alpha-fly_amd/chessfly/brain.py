@@ -259,7 +259,10 @@ def _pad_columns(batch: int, rows: int) -> int:
     two lines (full-size network, ms per forward and backward with rows of whole 16 bytes and of whole lines: 27
     positions 4.73 / 4.45, 36 5.08 / 4.97, 67 7.40 / 5.93, 68 6.29 / 5.45, 100 7.51 / 6.18, 145 10.99 / 7.88, 200
     11.27 / 8.71).  Below that rows of whole 16 bytes, since wider ones gain nothing (12 positions 4.15 / 4.33, 20 4.28 /
-    4.31).  A state that would pass 2 GiB is padded less, or not at all."""
+    4.31).  None behind a single position: the one-column products are the faster ones there (3.52 against 3.97).  A
+    state that would pass 2 GiB is padded less, or not at all."""
+    if batch == 1:
+        return 0
     for unit in (32, 4) if batch > 24 else (4,):
         pad = -batch % unit
         if rows * (batch + pad) * 4 < 2 ** 31:
