@@ -19,6 +19,7 @@
 // they are exact in float16 (binary planes always are); the split records that per board and a tile whose boards
 // are all exact leaves out the A_hi B_lo product.
 #include "common.hpp"
+#include "gemm_rules.hpp"
 
 #include <cmath>
 #include <cstring>
@@ -56,7 +57,7 @@ namespace {
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-constexpr int GBK = 64, LDK = GBK + 8;  // K per LDS stage; LDS rows padded to 144 bytes
+constexpr int LDK = GBK + 8;  // LDS rows of a stage padded to 144 bytes
 
 int64_t pad_k(int64_t k) { return round_up(std::max<int64_t>(k, 1), GBK); }
 
@@ -155,8 +156,8 @@ struct Split {
 // per element, a wave's stores covered four 64-byte pieces of four rows, and the encoder's 80 MB output took a
 // quarter of its time.
 struct EncoderEpilogue {
-  static constexpr bool kRows = true;
-  __device__ __forceinline__ EncoderEpilogue part(int) const { return *this; }   // its K loop is never split
+  static constexpr bool kRows = true, kParts = false;   // its K loop is never split
+  __device__ __forceinline__ EncoderEpilogue part(int) const { return *this; }
   const float *bias;
   float gain;
   float *u;
@@ -187,7 +188,7 @@ struct EncoderEpilogue {
 // ct[n, m] = C[m, n]: one row of all head outputs per board (measured: its element stores cost about 4 us), for each
 // part of a split K loop one after the other.
 struct HeadEpilogue {
-  static constexpr bool kRows = false;
+  static constexpr bool kRows = false, kParts = true;
   float *ct;
   int64_t ldc, part_stride;
   __device__ __forceinline__ HeadEpilogue part(int p) const { return {ct + p * part_stride, ldc, part_stride}; }
@@ -335,11 +336,16 @@ __global__ __launch_bounds__(256) void k_gemm_split(const Split A, const Split B
   auto As = reinterpret_cast<_Float16 (*)[32 * TM][LDK]>(smem);
   auto Bs = reinterpret_cast<_Float16 (*)[32 * TN][LDK]>(smem + 2 * LDK * 32 * TM);
   int ty, tx;
-  xcd_tile(tiles, gx * splits, ty, tx);
-  const int part = tx / gx;
-  tx -= part * gx;
-  const EP ep = whole.part(part);
-  const int64_t stages = kp / GBK, kbeg = stages * part / splits * GBK, kend = stages * (part + 1) / splits * GBK;
+  EP ep = whole;
+  int64_t kbeg = 0, kend = kp;
+  xcd_tile(tiles, EP::kParts ? gx * splits : gx, ty, tx);
+  if (EP::kParts && splits > 1) {   // the divisions cost 0.4 us of a head in one part
+    const int part = tx / gx, stages = (int)(kp / GBK);
+    tx -= part * gx;
+    ep = whole.part(part);
+    kbeg = stages * part / splits * GBK;
+    kend = stages * (part + 1) / splits * GBK;
+  }
   const int64_t m0 = (int64_t)ty * (32 * TM), n0 = (int64_t)tx * (32 * TN);
   bool blo = true;
   if (B.flag != nullptr) {  // uniform over the workgroup
@@ -352,40 +358,11 @@ __global__ __launch_bounds__(256) void k_gemm_split(const Split A, const Split B
     gemm_tile<TM, TN, false>(A, B, kp, kbeg, kend, unscale, ep, m0, n0, As, Bs);
 }
 
-// The workgroup tile, 10 TM + TN for 32 TM x 32 TN.  The gemm_tile tuning key forces one: 1 = 64 x 64, 2 = 128 x 64,
-// 3 = 128 x 128, or 10 TM + TN with TM in {2, 3, 4} and TN in {2, 4, 5}.  Otherwise, measured on the 17,937-row encoder
-// and the 4,299-row head (us):
-// * 128 x 128 from 1,024 tiles on: encoder of 1120 boards 106 against 121 (64 x 64) and 112 (64 x 160);
-// * 64 x 160 where its columns cover the batch with no more padding than 64 do and its tiles fill at least 82% of their
-//   rounds of 512 workgroups (two per CU): head of 1120 boards 125 against 129 (64 x 64), encoder of 480 60 against 68;
-//   with rounds less full it loses (head of 640: 103 against 87, of 1280: 167 against 147);
-// * 128 x 128 from 400 tiles on that pad at most 10% more columns than 64: head of 1500 boards 154 against 169, encoder
-//   of 640 73 against 77, but of 400 (512 columns against 448) 65 against 60;
-// * else 64 x 64.
-int gemm_shape(int64_t arows, int64_t brows, int tile_key) {
-  int shape = tile_key;
-  if (shape == 1) shape = 22;
-  else if (shape == 2) shape = 42;
-  else if (shape == 3) shape = 44;
-  const int tm = shape / 10, tn = shape % 10;
-  if ((tm == 2 || tm == 3 || tm == 4) && (tn == 2 || tn == 4 || tn == 5)) return shape;
-  const int64_t large = ((arows + 127) / 128) * ((brows + 127) / 128);
-  if (large >= 1024) return 44;
-  const int64_t wide = ((arows + 63) / 64) * ((brows + 159) / 160);
-  if (round_up(brows, 160) <= round_up(brows, 64) && wide * 100 >= round_up(wide, 512) * 82) return 25;
-  return large >= 400 && round_up(brows, 128) * 10 <= round_up(brows, 64) * 11 ? 44 : 22;
-}
-
-int64_t gemm_tiles(int64_t arows, int64_t brows, int shape) {
-  const int bm = 32 * (shape / 10), bn = 32 * (shape % 10);
-  return ((arows + bm - 1) / bm) * ((brows + bn - 1) / bn);
-}
-
 template <class EP>
 void gemm_split(const Split &A, const Split &B, int64_t kp, float unscale, const EP &ep, int tile_key, int splits,
                 hipStream_t st) {
   if (A.rows == 0 || B.rows == 0) return;
-  const int shape = gemm_shape(A.rows, B.rows, tile_key);
+  const int shape = gemm_shape(A.rows, B.rows, kp / GBK, tile_key);
   const int bn = 32 * (shape % 10);
   const int64_t gx = (B.rows + bn - 1) / bn, tiles = gemm_tiles(A.rows, B.rows, shape) * splits;
   FLY_REQUIRE(tiles < INT32_MAX, "GEMM grid too large");
@@ -416,7 +393,8 @@ void gemm_split(const Split &A, const Split &B, int64_t kp, float unscale, const
 // ct holds `parts` shares of C (a split K loop's), part_stride apart, added in order.
 // One workgroup per board: its from- and to-square terms (64 + 64 values plus biases) go to LDS once, then each
 // thread writes 4 consecutive moves with 16-byte loads and stores when `vec` (the move count and the rows allow
-// them), one move at a time otherwise.
+// them), one move at a time otherwise.  PARTS: more than one share (the loops over them cost 0.4 us where there is one).
+template <bool PARTS>
 __global__ __launch_bounds__(256) void k_assemble(const float *__restrict__ ct, int64_t ldc, int32_t parts,
                                                   int64_t part_stride, int64_t n_moves,
                                                   const float *__restrict__ b, const int32_t *__restrict__ mfrom,
@@ -427,7 +405,8 @@ __global__ __launch_bounds__(256) void k_assemble(const float *__restrict__ ct, 
     const float *row = ct + n * ldc;
     auto value = [&](int64_t i) {
       float v = row[i];
-      for (int32_t p = 1; p < parts; ++p) v += row[p * part_stride + i];
+      if constexpr (PARTS)
+        for (int32_t p = 1; p < parts; ++p) v += row[p * part_stride + i];
       return v;
     };
     __syncthreads();   // the previous board's squares are read
@@ -439,10 +418,11 @@ __global__ __launch_bounds__(256) void k_assemble(const float *__restrict__ ct, 
       for (int64_t i = 4 * (int64_t)threadIdx.x; i < n_moves; i += 4 * (int64_t)blockDim.x) {
         float4 p = *reinterpret_cast<const float4 *>(row + i);
         const float4 bp = *reinterpret_cast<const float4 *>(b + i);
-        for (int32_t q = 1; q < parts; ++q) {
-          const float4 w = *reinterpret_cast<const float4 *>(row + q * part_stride + i);
-          p = make_float4(p.x + w.x, p.y + w.y, p.z + w.z, p.w + w.w);
-        }
+        if constexpr (PARTS)
+          for (int32_t q = 1; q < parts; ++q) {
+            const float4 w = *reinterpret_cast<const float4 *>(row + q * part_stride + i);
+            p = make_float4(p.x + w.x, p.y + w.y, p.z + w.z, p.w + w.w);
+          }
         const int4 fr = *reinterpret_cast<const int4 *>(mfrom + i), to = *reinterpret_cast<const int4 *>(mto + i);
         *reinterpret_cast<float4 *>(out + i) =
             make_float4(((p.x + bp.x) + sq[fr.x]) + sq[64 + to.x], ((p.y + bp.y) + sq[fr.y]) + sq[64 + to.y],
@@ -527,23 +507,12 @@ size_t encoder_ws(const fly_dense &d, int64_t batch) {
   return 2 * split_bytes(batch, d.kp_enc) + align256((size_t)batch * sizeof(int32_t));
 }
 
-// Parts of the head GEMM's K loop.  Its 4,299 rows make few tiles (68 for up to 64 boards), each a chain of 37 stages;
-// parts of K fill the other CUs, at the cost of a share of C each (k_assemble adds them).  The fewest parts, up to 3,
-// within 15% of the least rounds of 512 workgroups (two per CU) per part; none past 640 tiles, where the shares' bytes
-// cost what the rounds gain.  Measured, us of the head for 1, 2 and 3 parts: 1 board 42 / 30 / 27 (6: 30, 8: 34), 128
-// boards 52 / 44 / 38, 256 boards 65 / 57 / 55, 480 boards 89 / 77 / 87, 640 boards 113 / 107 / 103, 1120 boards 125 /
-// 135 / 152.
+// Parts of the head GEMM's K loop for `batch` boards (head_parts, or the forced number where the stages allow it).
 int head_splits(const fly_dense &d, int64_t batch) {
   const int64_t stages = d.kp_head / GBK;
   if (d.gemm_splits > 0) return (int)std::min<int64_t>(d.gemm_splits, stages);
-  const int64_t tiles = gemm_tiles(d.head_rows(), batch, gemm_shape(d.head_rows(), batch, d.gemm_tile));
-  const int most = tiles > 640 ? 1 : (int)std::min<int64_t>(3, stages);
-  auto cost = [&](int s) { return (double)((tiles * s + 511) / 512) / s; };
-  double least = cost(1);
-  for (int s = 2; s <= most; ++s) least = std::min(least, cost(s));
-  int s = 1;
-  while (cost(s) > 1.15 * least) ++s;
-  return s;
+  const int shape = gemm_shape(d.head_rows(), batch, stages, d.gemm_tile);
+  return head_parts(gemm_tiles(d.head_rows(), batch, shape), stages);
 }
 
 // The head's scratch with `rows` rows of C (boards times parts).
@@ -594,9 +563,9 @@ void run_head(const fly_dense &d, const S *state, int64_t lds, const int32_t *sr
   gemm_split(Split{d.head_hi.p, d.head_lo.p, d.head_rows(), nullptr}, Split{rh, rl, batch, nullptr}, d.kp_head,
              d.head_unscale, HeadEpilogue{ct, ldc, batch * ldc}, d.gemm_tile, splits, st);
   const bool avec = d.n_moves % 4 == 0 && ldc % 4 == 0 && aligned(logits, 16);
-  hipLaunchKernelGGL(k_assemble, dim3((unsigned)std::min<int64_t>(batch, 65535)), dim3(256), 0, st, ct, ldc, splits,
-                     batch * ldc, d.n_moves,
-                     d.head_b.p, d.move_from.p, d.move_to.p, batch, avec, logits, wdl);
+  hipLaunchKernelGGL(splits > 1 ? k_assemble<true> : k_assemble<false>, dim3((unsigned)std::min<int64_t>(batch, 65535)),
+                     dim3(256), 0, st, ct, ldc, splits, batch * ldc, d.n_moves, d.head_b.p, d.move_from.p, d.move_to.p,
+                     batch, avec, logits, wdl);
   check_launch("head assembly");
 }
 
