@@ -67,14 +67,32 @@ inline int current_device() {
   return d;
 }
 
+// While one exists, its thread may free memory although a stream is being captured: a free outside this mode spoils every
+// capture that is not relaxed itself.
+class RelaxedCapture {
+ public:
+  RelaxedCapture() { ok_ = hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess; }
+  ~RelaxedCapture() {
+    if (ok_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+  }
+  RelaxedCapture(const RelaxedCapture &) = delete;
+  RelaxedCapture &operator=(const RelaxedCapture &) = delete;
+
+ private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;   // then the thread's own mode
+  bool ok_ = false;
+};
+
 // Device memory that objects have given back, kept for the next object's arrays: hipMalloc and hipFree of a plan's 300 MB
 // took 2.5 ms of the 5.5 ms between a new snapshot's arrival and its first answer (the maps and unmaps, and the waits
 // around them).  At most kMost bytes per device stay idle, and all of them go back to the runtime when the last array
 // of the process's library objects on that device is released, or when an allocation fails.
 //
 // A block is handed on only once no GPU work can still use it: alloc() waits for the device if the block came back
-// after the last such wait, unless a QuietRelease said then that its work was over.  Releasing makes no GPU call while
-// the block stays here (a wait there would spoil a stream capture, as hipFree does).  Safe to use from several threads.
+// after the last such wait, unless a QuietRelease said then that its work was over.  Releasing does not wait, and what
+// it gives back to the runtime it frees under RelaxedCapture, so an object may go away while a stream is being captured.
+// The wait is hipFree's own: hipDeviceSynchronize refuses, and spoils every capture of the process, in whatever mode.
+// Where even that fails the block stays idle and alloc() takes new memory.  Safe to use from several threads.
 class DevicePool {
  public:
   static DevicePool &get() {
@@ -84,33 +102,8 @@ class DevicePool {
   // `device`: the current one.
   void *alloc(size_t bytes, int device) {
     bytes = rounded(bytes);
+    if (void *p = take(bytes, device)) return p;
     void *p = nullptr;
-    bool wait = false;
-    uint64_t upto = 0;   // a wait that starts now covers the blocks that came back as number 1 .. upto
-    {
-      std::lock_guard<std::mutex> lock(mu_);
-      Device &d = devices_[device];
-      const auto best = d.idle.lower_bound(bytes);   // the smallest that holds it
-      if (best != d.idle.end() && best->first <= bytes + bytes / 4) {
-        p = best->second.p;
-        wait = best->second.back > d.waited;
-        upto = d.back;
-        sizes_[p] = best->first;
-        d.idle_bytes -= best->first;
-        d.idle.erase(best);
-        ++d.live;
-      }
-    }
-    if (p && wait) {
-      if (const hipError_t e = hipDeviceSynchronize(); e != hipSuccess) {
-        (void)hipGetLastError();
-        free(p, device, false);
-        FLY_HIP(e);
-      }
-      std::lock_guard<std::mutex> lock(mu_);
-      devices_[device].waited = std::max(devices_[device].waited, upto);
-    }
-    if (p) return p;
     if (hipMalloc(&p, bytes) != hipSuccess) {
       (void)hipGetLastError();
       trim(device);
@@ -138,7 +131,17 @@ class DevicePool {
       }
       if (--d.live == 0) take_idle(d, give);
     }
-    for (void *q : give) (void)hipFree(q);   // waits for the device itself
+    give_back(give);
+  }
+  // Gives the idle blocks of `device` (-1: of every device) back to the runtime.
+  void trim(int device) {
+    std::vector<void *> give;
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      for (auto &e : devices_)
+        if (device < 0 || e.first == device) take_idle(e.second, give);
+    }
+    give_back(give);
   }
 
  private:
@@ -158,18 +161,57 @@ class DevicePool {
     const size_t unit = bytes >= ((size_t)1 << 20) ? (size_t)2 << 20 : 4096;
     return (bytes + unit - 1) / unit * unit;
   }
+  // An idle block of at least `bytes`, the smallest that holds them and wastes little, or null.
+  void *take(size_t bytes, int device) {
+    size_t size = 0;
+    Block block{};
+    uint64_t upto = 0;   // a wait that starts now covers the blocks that came back as number 1 .. upto
+    bool wait = false;
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      Device &d = devices_[device];
+      const auto best = d.idle.lower_bound(bytes);
+      if (best == d.idle.end() || best->first > bytes + bytes / 4) return nullptr;
+      size = best->first;
+      block = best->second;
+      wait = block.back > d.waited;
+      upto = d.back;
+      sizes_[block.p] = size;
+      d.idle_bytes -= size;
+      d.idle.erase(best);
+      ++d.live;
+    }
+    if (!wait) return block.p;
+    const bool waited = wait_for_device();
+    std::lock_guard<std::mutex> lock(mu_);
+    Device &d = devices_[device];
+    if (waited) {
+      d.waited = std::max(d.waited, upto);
+      return block.p;
+    }
+    sizes_.erase(block.p);
+    d.idle.emplace(size, block);   // idle as before, with its number
+    d.idle_bytes += size;
+    --d.live;
+    return nullptr;
+  }
+  // Waits until the current device has no work left: hipFree does, before it frees.
+  static bool wait_for_device() {
+    RelaxedCapture relaxed;
+    void *p = nullptr;
+    if (hipMalloc(&p, 4096) == hipSuccess && hipFree(p) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+  }
   static void take_idle(Device &d, std::vector<void *> &out) {
     for (const auto &e : d.idle) out.push_back(e.second.p);
     d.idle.clear();
     d.idle_bytes = 0;
   }
-  void trim(int device) {
-    std::vector<void *> give;
-    {
-      std::lock_guard<std::mutex> lock(mu_);
-      take_idle(devices_[device], give);
-    }
-    for (void *q : give) (void)hipFree(q);
+  static void give_back(const std::vector<void *> &blocks) {
+    if (blocks.empty()) return;
+    RelaxedCapture relaxed;
+    for (void *p : blocks) (void)hipFree(p);   // waits for the device itself
   }
   std::mutex mu_;
   std::map<int, Device> devices_;

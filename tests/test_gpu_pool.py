@@ -4,6 +4,8 @@ the right answers."""
 
 from __future__ import annotations
 
+import ctypes
+import gc
 import threading
 
 import numpy as np
@@ -13,6 +15,7 @@ import torch
 from helpers import brain_arrays, random_params
 from test_gpu_sweep import _cone, _medium, _rnn
 
+from chessfly import _hip
 from oracle import forward as F
 
 pytestmark = pytest.mark.gpu
@@ -69,3 +72,84 @@ def test_threads_build_and_destroy_at_once():
     for t in threads:
         t.join()
     assert not failed, failed
+
+
+def _captured(inside, mode="global"):
+    """Captures two operations with inside() between them, and replays them."""
+    x = torch.ones(1000, device=DEV)
+    gc.collect()                                         # what earlier tests left goes away now
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, capture_error_mode=mode):
+        y = x * 2
+        inside()
+        z = y + 1
+    for i in range(3):
+        x.fill_(float(i))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float(z[0]) == 2.0 * i + 1 and bool((z == z[0]).all())
+
+
+def test_objects_released_while_a_graph_is_captured():
+    """A network that goes away while a graph is being captured leaves the capture as it is, and the next network gets the
+    right answers."""
+    conn, (lg, b, al), ind, outd, u, ref = _case(7, 64)
+    nets = [_rnn(conn, 4.0, lg, b, al), _rnn(conn, 4.0, lg, b, al)]
+    with torch.no_grad():
+        for i in range(2):
+            nets[i].forward_io(u, ind, outd, 4)
+
+        def drop():
+            nets.pop()
+            gc.collect()
+
+        _captured(drop)
+        for rnn in (nets[0], _rnn(conn, 4.0, lg, b, al)):
+            out = rnn.forward_io(u, ind, outd, 4).cpu().numpy()
+            np.testing.assert_allclose(out, ref, rtol=2e-5, atol=2e-5 * max(np.abs(ref).max(), 1.0))
+
+
+def test_more_than_stays_idle_is_released_while_a_graph_is_captured():
+    """Plans of 800 MB destroyed during a capture, beside one that lives on: what is past the bound goes back to the runtime
+    at once."""
+    lib = _hip.load()
+    n, per = 2_000_000, 8
+    crow = torch.arange(0, n + 1, dtype=torch.int32, device=DEV) * per
+    pre = (torch.arange(n * per, dtype=torch.int32, device=DEV) * 7) % n
+    w, al = torch.ones(n * per, device=DEV), torch.zeros(n, device=DEV)
+    plans = []
+    for _ in range(5):                                   # 200 MB each
+        h = ctypes.c_void_p()
+        _hip.check(lib.fly_plan_create_full(n, n * per, crow.data_ptr(), pre.data_ptr(), w.data_ptr(), al.data_ptr(), 10.0,
+                                            None, _hip.stream(w.device), ctypes.byref(h)), "fly_plan_create_full")
+        plans.append(h)
+    del crow, pre, w, al
+    _captured(lambda: [_hip.check(lib.fly_plan_destroy(h), "fly_plan_destroy") for h in plans[1:]])
+    _hip.check(lib.fly_plan_destroy(plans[0]), "fly_plan_destroy")
+
+
+@pytest.mark.parametrize("mode", ["thread_local", "relaxed"])
+def test_another_thread_builds_while_a_graph_is_captured(mode):
+    """A network built on another thread, out of memory that must be waited for, while this one captures."""
+    conn, (lg, b, al), ind, outd, u, ref = _case(8, 64)
+    with torch.no_grad():
+        keep = _rnn(conn, 4.0, lg, b, al)
+        keep.forward_io(u, ind, outd, 4)
+        _rnn(conn, 4.0, lg, b, al).forward_io(u, ind, outd, 4)        # goes away: its memory is handed on below
+        fresh = _rnn(conn, 4.0, lg, b, al)
+    got = []
+
+    def build():
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream), torch.no_grad():
+            got.append(fresh.forward_io(u, ind, outd, 4))
+            stream.synchronize()
+
+    def other():
+        thread = threading.Thread(target=build)
+        thread.start()
+        thread.join()
+
+    _captured(other, mode)
+    np.testing.assert_allclose(got[0].cpu().numpy(), ref, rtol=2e-5, atol=2e-5 * max(np.abs(ref).max(), 1.0))
