@@ -37,6 +37,7 @@ class HeadDesc(ctypes.Structure):
 SIGNATURES = {
     "fly_abi_version": (_i32, []),
     "fly_last_error": (ctypes.c_char_p, []),
+    "fly_trim_memory": (_i32, []),
     "fly_cone_create": (_i32, [_i64, _i64, _p, _p, _p, _i64, _p, _i64, _i32, _i32, _p, _pp]),
     "fly_cone_destroy": (_i32, [_p]),
     "fly_cone_sizes": (_i32, [_p, _p, _p, _p]),
@@ -146,6 +147,11 @@ def ptr(t: torch.Tensor | None) -> int | None:
 def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     """Scratch bytes from torch's caching allocator (256-byte aligned by construction)."""
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
+
+
+def trim_memory() -> None:
+    """Give the device memory that the library keeps idle for its next objects back to the runtime (fly_trim_memory)."""
+    check(load().fly_trim_memory(), "fly_trim_memory")
 
 
 KERNEL_CLASSES = ("state_step", "encoder", "head", "other")

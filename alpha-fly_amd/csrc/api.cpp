@@ -77,6 +77,10 @@ extern "C" int fly_abi_version(void) { return FLY_ABI_VERSION; }
 
 extern "C" const char *fly_last_error(void) { return fly::g_last_error.c_str(); }
 
+extern "C" int fly_trim_memory(void) {
+  return guard([] { DevicePool::get().trim(-1); });
+}
+
 extern "C" int fly_profile_enable(int32_t on) {
   return guard([&] {
     Profiler &p = profiler();

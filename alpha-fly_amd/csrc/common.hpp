@@ -86,7 +86,7 @@ class RelaxedCapture {
 // Device memory that objects have given back, kept for the next object's arrays: hipMalloc and hipFree of a plan's 300 MB
 // took 2.5 ms of the 5.5 ms between a new snapshot's arrival and its first answer (the maps and unmaps, and the waits
 // around them).  At most kMost bytes per device stay idle, and all of them go back to the runtime when the last array
-// of the process's library objects on that device is released, or when an allocation fails.
+// of the process's library objects on that device is released, when an allocation fails, or by fly_trim_memory.
 //
 // A block is handed on only once no GPU work can still use it: alloc() waits for the device if the block came back
 // after the last such wait, unless a QuietRelease said then that its work was over.  Releasing does not wait, and what

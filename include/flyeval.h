@@ -78,6 +78,13 @@ typedef struct fly_sweep fly_sweep;
 int fly_abi_version(void);
 const char *fly_last_error(void);
 
+/* The device memory of destroyed objects stays with the library for the next objects' arrays: at most 512 MiB per
+ * device, until the last object of the process on that device is destroyed, an allocation of the library fails, or
+ * this call gives all of it back to the runtime (it waits for the devices).  Other allocators of the process cannot
+ * reach that memory: a program that runs short of it calls this.  An object may be destroyed while a stream is being
+ * captured; not so the call itself. */
+int fly_trim_memory(void);
+
 /* ---- light cone (integer, bit-exact with chessfly/brain.py:126-173) ------------------------------
  * crow_dev (n+1), pre_dev (n_edges): CSR of W; in_idx_dev (n_in), out_idx_dev (n_out): neuron ids.
  * flags: 0 prunes to the light cone; FLY_CONE_UNPRUNED computes every neuron at every step t >= 1 (the

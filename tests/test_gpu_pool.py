@@ -112,7 +112,7 @@ def test_objects_released_while_a_graph_is_captured():
 
 def test_more_than_stays_idle_is_released_while_a_graph_is_captured():
     """Plans of 800 MB destroyed during a capture, beside one that lives on: what is past the bound goes back to the runtime
-    at once."""
+    at once, the rest stays idle until it is asked for."""
     lib = _hip.load()
     n, per = 2_000_000, 8
     crow = torch.arange(0, n + 1, dtype=torch.int32, device=DEV) * per
@@ -126,7 +126,12 @@ def test_more_than_stays_idle_is_released_while_a_graph_is_captured():
         plans.append(h)
     del crow, pre, w, al
     _captured(lambda: [_hip.check(lib.fly_plan_destroy(h), "fly_plan_destroy") for h in plans[1:]])
+    torch.cuda.empty_cache()
+    held = torch.cuda.mem_get_info()[0]
+    _hip.trim_memory()
+    back = torch.cuda.mem_get_info()[0] - held
     _hip.check(lib.fly_plan_destroy(plans[0]), "fly_plan_destroy")
+    assert (200 << 20) < back <= (512 << 20), back       # what stayed idle, and no more than the bound
 
 
 @pytest.mark.parametrize("mode", ["thread_local", "relaxed"])
