@@ -33,20 +33,39 @@ def _case(seed, batch):
 
 
 def test_new_weight_versions_on_two_streams():
-    """Forwards of ten weight versions alternate between two streams with no wait in between: each new plan destroys the
-    one that the other stream may still be running."""
-    conn, (lg, b, al), ind, outd, u, ref = _case(3, 256)
+    """Forwards of six weight versions alternate between two streams with no wait in between, each behind some 20 ms of
+    other work: a new version's plan destroys the old one while its forward is still pending on the other stream, and
+    takes arrays of the same sizes.  Every version has weights of its own and is checked against its own float64
+    reference, so arrays handed on too early give a wrong answer."""
+    conn, (lg, b, al), ind, outd, u, _ = _case(3, 256)
+    versions = [(lg + np.float32(0.1 * i), b + np.float32(0.05 * i), al) for i in range(6)]
+    cone = _cone(conn, conn.nodes("afferent"), conn.nodes("efferent"), 4)
+    refs = [F.cone_f32(brain_arrays(conn, 4.0, *v, dtype=torch.float64), cone, u.cpu().double(), 4).numpy() for v in versions]
+    for x, y in zip(refs, refs[1:]):
+        assert np.abs(x - y).max() > 1e-2 * np.abs(x).max()
     rnn = _rnn(conn, 4.0, lg, b, al)
+    params = [[torch.as_tensor(p).to(DEV) for p in v] for v in versions]
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
-    outs = []
-    torch.cuda.synchronize()
+    m = torch.randn(8192, 8192, device=DEV)
+    outs, done, pending = [], [], 0
     with torch.no_grad():
-        for i in range(10):
+        rnn.forward_io(u, ind, outd, 4)                  # the cone
+        torch.cuda.synchronize()
+        for i, v in enumerate(params):
             with torch.cuda.stream(streams[i % 2]):
-                rnn.bias.add_(0.0)                       # a new version of the same values
+                for p, new in zip((rnn.log_gain, rnn.bias, rnn.alpha_logit), v):
+                    p.copy_(new)                         # no forward reads them: a plan holds what it needs
+                pending += int(bool(done) and not done[-1].query())
+                plan = rnn._cone_plan(rnn.light_cone(ind, outd, 4), 1)
+                for _ in range(2):
+                    m @ m
                 outs.append(rnn.forward_io(u, ind, outd, 4))
+                assert rnn._cone_plan(rnn.light_cone(ind, outd, 4), 1) is plan
+                done.append(torch.cuda.Event())
+                done[-1].record()
     torch.cuda.synchronize()
-    for out in outs:
+    assert pending == len(params) - 1                    # every plan was destroyed ahead of its forward's end
+    for out, ref in zip(outs, refs):
         np.testing.assert_allclose(out.cpu().numpy(), ref, rtol=2e-5, atol=2e-5 * max(np.abs(ref).max(), 1.0))
 
 
