@@ -270,7 +270,10 @@ extern "C" int fly_plan_create(const fly_cone *cone, const int32_t *crow, const 
                              cone->edge[t].p, w, cone->nnz[t], plan->colval[t].p);
         if (plan->tune.swept >= 0) {
           plan->sweep[t] = cone_sweep(*cone, t, cfg, st);
-          if (plan->sweep[t]) plan->max_pieces = std::max(plan->max_pieces, plan->sweep[t]->pieces);
+          if (plan->sweep[t]) {
+            plan->max_pieces = std::max(plan->max_pieces, plan->sweep[t]->pieces);
+            if (narrow_on(plan->tune)) need_stage(cone->rowptr[t].p, cone->col[t].p, *plan->sweep[t], st);
+          }
         }
         if (cone->nnz[t] < 16 * nr) {   // short rows on average: the step runs as row slots
           LeadSlots ls = build_lead_slots(plan->rowptr[t].p, nr, cone->nnz[t], st);
@@ -356,6 +359,7 @@ extern "C" int fly_plan_create_full(int64_t n, int64_t n_edges, const int32_t *c
                   "the sweep tables belong to another structure");
       plan->sweep[0] = sweep->t;
       plan->max_pieces = sweep->t->pieces;
+      if (narrow_on(plan->tune)) need_stage(crow, pre, *sweep->t, st);
     }
     check_launch("full plan");
     FLY_HIP(hipStreamSynchronize(st));

@@ -73,11 +73,6 @@ void launch_v(const StepArgs<S, U> &a, int groups, int unroll, bool rows_mode, i
     hipLaunchKernelGGL((k_state_step<S, U, V, 8, kTL>), grid, block, lds, st, a);
 }
 
-// Whether steps of a plan created under `tune` may run narrow: not where a key asks for another kernel's shape.
-bool narrow_on(const Tuning &tune) {
-  return tune.narrow >= 0 && tune.swept <= 0 && tune.vec == 0 && tune.groups == 0 && tune.rows_mode == 0;
-}
-
 // The narrow kernel for batches of up to 32 bytes a row, where the rows' 16-byte (2- or 4-byte) pieces can be read.
 template <typename S, typename U, int V, int L>
 void launch_narrow(StepArgs<S, U> &a, const Tuning &tune, hipStream_t st) {

@@ -67,8 +67,18 @@ struct SweepTables {
   DevArray<int32_t> split;          // (split_rows): the rows split into pieces
   DevArray<int32_t> split_ptr;      // (split_rows + 1): the pieces of split[h] are split_ptr[h] .. split_ptr[h + 1] - 1
   DevArray<int32_t> piece_row;      // (pieces): the row each piece belongs to
-  StageTables stage[2];             // for state rows of 2 and of 4 bytes
+  // The staged step's tables, for state rows of 2 and of 4 bytes: built on the first plan whose steps may take them
+  // (need_stage, under the lock) and never changed after that.
+  mutable std::mutex stage_mu;
+  mutable bool stage_built = false;
+  mutable StageTables stage[2];
 };
+
+// Whether steps of a plan created under `tune` may run narrow, and staged: not where a key asks for another kernel's
+// shape.
+inline bool narrow_on(const Tuning &tune) {
+  return tune.narrow >= 0 && tune.swept <= 0 && tune.vec == 0 && tune.groups == 0 && tune.rows_mode == 0;
+}
 
 // The GPU's CU count (the swept kernel runs one workgroup per CU), per device, cached; safe to call from several
 // threads (a first call that races computes the same value).
@@ -479,35 +489,6 @@ __global__ void k_sweep_ranges(const int32_t *__restrict__ off, int K, int64_t n
   }
 }
 
-// The staged step's tables of t's structure: none where its columns are out of order, or where a forced sweep's matrix is
-// so small that its bands' sums outgrow their place behind the state rows or a band holds no whole 16-byte piece.
-template <typename C>
-void build_stage(const int32_t *rowptr, const C *cols, SweepTables &t, hipStream_t st) {
-  if (t.nrows < 64 || t.ncols < 64) return;
-  DevArray<int32_t> bad(1);
-  const int32_t zero = 0;
-  FLY_HIP(hipMemcpyAsync(bad.p, &zero, sizeof(zero), hipMemcpyHostToDevice, st));
-  for (int i = 0; i < 2; ++i) {
-    const int64_t most = (kStageBytes / (2 << i) - 1) / 64 * 64, bands = (t.ncols + most - 1) / most;
-    if (bands > kStageBands) continue;
-    StageTables &s = t.stage[i];
-    s.bands = (int32_t)bands;
-    s.band_rows = (int32_t)round_up((t.ncols + bands - 1) / bands, 64);   // 64 rows: every band starts on a line
-    s.start.alloc((size_t)(bands + 1) * t.nrows);
-    hipLaunchKernelGGL(k_stage_starts<C>, dim3(blocks_for(t.nrows, 16)), dim3(256), 0, st, rowptr, cols, t.nrows,
-                       t.ncols, s.bands, s.band_rows, s.start.p, bad.p);
-  }
-  check_launch("stage tables");
-  int32_t wrong = 0;
-  FLY_HIP(hipMemcpyAsync(&wrong, bad.p, sizeof(wrong), hipMemcpyDeviceToHost, st));
-  FLY_HIP(hipStreamSynchronize(st));
-  if (!wrong) return;
-  for (StageTables &s : t.stage) {
-    s.bands = 0;
-    s.start.release();
-  }
-}
-
 }  // namespace
 
 // The tables of one CSR structure (rowptr nrows + 1, records or columns nnz, columns below ncols), or null when it
@@ -696,9 +677,44 @@ std::shared_ptr<SweepTables> build_sweep(const int32_t *rowptr, const C *cols, i
     check_launch("sweep order");
     FLY_HIP(hipStreamSynchronize(st));
   }
-  build_stage<C>(rowptr, cols, *t, st);
   FLY_HIP(hipStreamSynchronize(st));
   return t;
+}
+
+// Builds the staged step's tables of t's structure (rowptr, cols: the arrays t was built from) where no earlier call has:
+// training's products and the probes never read them.  None where the columns are out of order, or where the matrix is so
+// small that its bands' sums outgrow their place behind the state rows or a band holds no whole 16-byte piece.
+// Synchronises the stream.
+inline void need_stage(const int32_t *rowptr, const int32_t *cols, const SweepTables &t, hipStream_t st) {
+  std::lock_guard<std::mutex> lock(t.stage_mu);
+  if (t.stage_built) return;
+  if (t.nrows >= 64 && t.ncols >= 64) {
+    StageTables made[2];
+    DevArray<int32_t> bad(1);
+    const int32_t zero = 0;
+    FLY_HIP(hipMemcpyAsync(bad.p, &zero, sizeof(zero), hipMemcpyHostToDevice, st));
+    for (int i = 0; i < 2; ++i) {
+      const int64_t most = (kStageBytes / (2 << i) - 1) / 64 * 64, bands = (t.ncols + most - 1) / most;
+      if (bands > kStageBands) continue;
+      StageTables &s = made[i];
+      s.bands = (int32_t)bands;
+      s.band_rows = (int32_t)round_up((t.ncols + bands - 1) / bands, 64);   // 64 rows: every band starts on a line
+      s.start.alloc((size_t)(bands + 1) * t.nrows);
+      hipLaunchKernelGGL(k_stage_starts<int32_t>, dim3(blocks_for(t.nrows, 16)), dim3(256), 0, st, rowptr, cols, t.nrows,
+                         t.ncols, s.bands, s.band_rows, s.start.p, bad.p);
+    }
+    check_launch("stage tables");
+    int32_t wrong = 0;
+    FLY_HIP(hipMemcpyAsync(&wrong, bad.p, sizeof(wrong), hipMemcpyDeviceToHost, st));
+    FLY_HIP(hipStreamSynchronize(st));
+    QuietRelease quiet;   // used on this stream only
+    bad.release();
+    if (!wrong)
+      for (int i = 0; i < 2; ++i) t.stage[i] = std::move(made[i]);
+    else
+      for (StageTables &s : made) s.start.release();
+  }
+  t.stage_built = true;
 }
 
 // The configuration of a plan's or fly_sweep's tables from its tuning (the order is searched for passes of two

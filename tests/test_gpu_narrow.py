@@ -36,12 +36,19 @@ def test_narrow_batches_match_the_oracle(batch):
     np.testing.assert_allclose(h.cpu().numpy(), ref, rtol=2e-5, atol=2e-5 * np.abs(ref).max())
 
 
-@pytest.fixture(scope="module")
-def staged_net():
-    """70,001 neurons (no multiple of a row quad) of 36 partners on average: enough rows, sources and partners to be
-    staged.  The first and last rows are empty, some hold 33, 96 and 97 partners and three are hubs of thousands."""
+def _kernels(call):
+    """call()'s result, and the names of the kernels that it launched."""
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        out = call()
+        torch.cuda.synchronize()
+    return out, " ".join(e.key for e in prof.key_averages())
+
+
+def _staged_conn(n):
+    """n neurons (no multiple of a row quad) of 36 partners on average: enough rows, sources and partners to be staged.
+    The first and last rows are empty, some hold 33, 96 and 97 partners and three are hubs of thousands."""
     from chessfly.synthetic import degree_connectome
-    n = 70_001
     rng = np.random.default_rng(5)
     deg = rng.poisson(36, n)
     deg[[0, 1, n - 1]] = 0
@@ -49,7 +56,12 @@ def staged_net():
     deg[[5, 40_000, n - 2]] = [20_000, 9_193, 3_000]
     ids = rng.permutation(n)
     conn = degree_connectome(deg, np.sort(ids[:500]), np.sort(ids[500:700]), seed=6)
-    lg, b, al = random_params(conn, 4, gain_sd=0.1)
+    return conn, random_params(conn, 4, gain_sd=0.1)
+
+
+@pytest.fixture(scope="module")
+def staged_net():
+    conn, (lg, b, al) = _staged_conn(70_001)
     return conn, _rnn(conn, 4.0, lg, b, al), brain_arrays(conn, 4.0, lg, b, al, dtype=torch.float64)
 
 
@@ -62,3 +74,19 @@ def test_staged_steps_match_the_oracle(staged_net, batch, dtype):
     ref = F.literal(ba, u.double(), 3).numpy()
     tol = 2e-5 if dtype == torch.float32 else 4e-3
     np.testing.assert_allclose(h.double().cpu().numpy(), ref, rtol=0, atol=tol * np.abs(ref).max())
+
+
+def test_stage_tables_are_built_for_plans_only():
+    """Training's products sweep the same structures and never read them."""
+    from chessfly import _hip
+    conn, (lg, b, al) = _staged_conn(70_001)
+    rnn = _rnn(conn, 4.0, lg, b, al)
+    u = torch.zeros(conn.n_neurons, 1, device=DEV)
+    with torch.no_grad():
+        tables, kernels = _kernels(lambda: _hip.sweep_create(rnn.crow32, rnn.pre32, rnn.n, rnn.n))
+        assert tables is not None and "k_band_off" in kernels and "k_stage_starts" not in kernels, kernels
+        _, kernels = _kernels(lambda: rnn(u, 2))
+        assert "k_stage_starts" in kernels, kernels
+        rnn.bias.add_(0.0)                                      # another weight version of the same structure
+        _, kernels = _kernels(lambda: rnn(u, 2))
+        assert "k_stage_sums" in kernels and "k_stage_starts" not in kernels, kernels
