@@ -59,9 +59,10 @@ def _staged_conn(n):
     return conn, random_params(conn, 4, gain_sd=0.1)
 
 
-@pytest.fixture(scope="module")
-def staged_net():
-    conn, (lg, b, al) = _staged_conn(70_001)
+@pytest.fixture(scope="module", params=[70_001, 150_001])
+def staged_net(request):
+    """Graphs whose states of 2 bytes a row take 1 and 3 bands of LDS, and of 4 bytes 2 and 5."""
+    conn, (lg, b, al) = _staged_conn(request.param)
     return conn, _rnn(conn, 4.0, lg, b, al), brain_arrays(conn, 4.0, lg, b, al, dtype=torch.float64)
 
 
@@ -70,8 +71,38 @@ def test_staged_steps_match_the_oracle(staged_net, batch, dtype):
     conn, rnn, ba = staged_net
     u = torch.randn(conn.n_neurons, batch, generator=torch.Generator().manual_seed(batch)).to(dtype)
     with torch.no_grad():
-        h = rnn(u.clone().to(DEV), 3)
+        h, kernels = _kernels(lambda: rnn(u.clone().to(DEV), 3))
+    assert "k_stage_sums" in kernels, kernels
     ref = F.literal(ba, u.double(), 3).numpy()
+    tol = 2e-5 if dtype == torch.float32 else 4e-3
+    np.testing.assert_allclose(h.double().cpu().numpy(), ref, rtol=0, atol=tol * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("batch", [1, 2])
+def test_staged_steps_of_the_light_cone_match_the_oracle(staged_net, batch):
+    """Enough steps for the cone to reach every neuron: its middle steps are staged in both state types at one position, in
+    half columns at two."""
+    conn, rnn, ba = staged_net
+    ind, outd = conn.nodes("afferent").to(DEV), conn.nodes("efferent").to(DEV)
+    u = torch.randn(len(ind), batch, generator=torch.Generator().manual_seed(batch))
+    with torch.no_grad():
+        for dtype in (torch.float16, torch.float32):
+            _, kernels = _kernels(lambda: rnn.forward_io(u.to(DEV, dtype), ind, outd, 8))
+            assert ("k_stage_sums" in kernels) == (batch * dtype.itemsize <= 4), kernels
+    _forward_io_both(rnn, conn, ba, batch, 8, batch, "auto")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_staged_steps_of_unbounded_activity_match_the_oracle(dtype):
+    conn, (lg, b, al) = _staged_conn(70_001)
+    rnn = _rnn(conn, 0.5, lg, b + 20.0, al, h_max=None)       # activities past the bound that there would be
+    ba = brain_arrays(conn, 0.5, lg, b + 20.0, al, h_max=float("inf"), dtype=torch.float64)
+    u = torch.randn(conn.n_neurons, 1, generator=torch.Generator().manual_seed(1)).to(dtype)
+    with torch.no_grad():
+        h, kernels = _kernels(lambda: rnn(u.clone().to(DEV), 3))
+    assert "k_stage_sums" in kernels, kernels
+    ref = F.literal(ba, u.double(), 3).numpy()
+    assert np.abs(ref).max() > 15
     tol = 2e-5 if dtype == torch.float32 else 4e-3
     np.testing.assert_allclose(h.double().cpu().numpy(), ref, rtol=0, atol=tol * np.abs(ref).max())
 
