@@ -22,7 +22,7 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("batch", [1, 2, 3, 4, 8, 9, 16, 17, 32, 33])
+@pytest.mark.parametrize("batch", [1, 2, 3, 4, 5, 8, 9, 12, 16, 17, 32, 33])
 def test_narrow_batches_match_the_oracle(batch):
     conn = _heavy_tailed(3)
     lg, b, al = random_params(conn, 9, gain_sd=0.1)
@@ -32,8 +32,11 @@ def test_narrow_batches_match_the_oracle(batch):
     u = torch.randn(conn.n_neurons, batch, generator=torch.Generator().manual_seed(batch))
     with torch.no_grad():
         h = rnn(u.clone().to(DEV), 4)
+        h16 = rnn(u.half().to(DEV), 4)
     ref = F.literal(ba, u.double(), 4).numpy()
     np.testing.assert_allclose(h.cpu().numpy(), ref, rtol=2e-5, atol=2e-5 * np.abs(ref).max())
+    ref = F.literal(ba, u.half().double(), 4).numpy()
+    np.testing.assert_allclose(h16.double().cpu().numpy(), ref, rtol=0, atol=4e-3 * np.abs(ref).max())
 
 
 def _kernels(call):
