@@ -284,7 +284,7 @@ inline int64_t state_ld(int64_t batch, size_t elem) {
   return ld;
 }
 
-// Row stride of a narrow batch's state buffer: the batch in 2, 4 or 16, 32 or 64 bytes, 0 for a wider batch.
+// Row stride of a narrow batch's state buffer: the batch in 2, 4, 16, 32 or 64 bytes, 0 for a wider batch.
 inline int64_t narrow_ld(int64_t batch, size_t elem) {
   for (int64_t bytes : {2, 4, 16, 32, 64})
     if (batch * (int64_t)elem <= bytes) return bytes / (int64_t)elem;
@@ -366,7 +366,7 @@ struct Tuning {
   int sweep_slots = 0;   // swept passes of 3 slots: 3 always, 0 when a wave owns 24 rows or fewer (else 6)
   int sweep_pipe = 0;    // swept gathers of the next four rounds in flight: 0 with 3 slots, 1 also 6, -1 never
   int nt_load = 0;       // read the carried state with non-temporal loads
-  int narrow = 0;        // batches of up to 64 bytes a row on the narrow kernel and state rows: 0 yes, -1 no
+  int narrow = 0;        // batches of up to 64 bytes a row on narrow state rows, up to 32 on the narrow kernel: 0 yes, -1 no
   int sweep_last_sync = 0;  // 1: a swept workgroup also meets after the last band of a chunk
 };
 // A copy of the current defaults (taken under a lock: fly_set_tuning may run on another thread).

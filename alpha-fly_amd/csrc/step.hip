@@ -109,8 +109,12 @@ void launch_staged(StepArgs<S, U> &a, const StageTables &t, const Tuning &tune, 
 // Why the lines lie there (full-size network, us per forward, before and after): 1 position 397 -> 190 staged, 2
 // positions 397 -> 195 staged, 3 to 8 397 -> 275 narrow, 9 to 16 397 -> 335 narrow.  At 17 to 32 positions (64 bytes a
 // row) the narrow kernel took 426 against 399, since its 10.7 MB of source rows overflow an XCD's L2; there the wide
-// kernels run on 64-byte state rows (387: half the lines of a band).  Staged rows of 8 bytes would serve 4 positions, but
-// a board would then sum in another order at 4 positions than at 5.
+// kernels run on 64-byte state rows (387: half the lines of a band).  Staged rows of 8 bytes (4 half columns, 2 float) are
+// untried.
+// Hub rows, which the wide kernels split or start first, are not split here, and cost less than the rest gains.  The
+// recurrence alone, wide kernels and here: in-degrees alike among neighbours, up to 9,193 partners, float16, 3 positions
+// 412 -> 247, 8 406 -> 248, 16 406 -> 268, float32, 4 positions 376 -> 243, 8 376 -> 268; a connectome's in-degrees,
+// float16, 1 position 497 -> 230 (staged), 3 499 -> 377, 8 494 -> 377, 16 493 -> 395, float32, 8 positions 451 -> 406.
 template <typename S, typename U>
 bool narrow_step(StepArgs<S, U> &a, const Tuning &tune, const SweepTables *sweep, hipStream_t st) {
   constexpr int E = (int)sizeof(S), V = 16 / E;
@@ -324,8 +328,8 @@ size_t io_workspace(const fly_plan &plan, int64_t batch) {
   return io_states_bytes(plan, blk) + plan_pieces_bytes(plan, blk);
 }
 
-// The two state buffers (rows, ld) at ws, each on a 256-byte boundary, and the scratch of the staged steps' band sums
-// after them for rows of up to 4 bytes (null otherwise).  All of it lies inside the space of two state_ld buffers:
+// The two state buffers (rows, ld) at ws, and after them the scratch of the staged steps' band sums for rows of up to 4
+// bytes (null otherwise).  The second buffer starts on 256 bytes for such rows, and on 16, as its rows do, for wider ones.  All of it lies inside the space of two state_ld buffers:
 // those hold at least 128 bytes a row, of which two narrow rows and kStageBands sums of each of their columns take
 // at most 72.
 template <typename S>

@@ -699,12 +699,13 @@ __device__ __forceinline__ float narrow_sum(const float (&acc)[V], int lane) {
 }
 
 // A step of a batch whose state rows hold L pieces of V columns (one piece of 2, 4 or 16 bytes, or 2 of 16: up to 16
-// half or 8 float columns).  16 ways of L lanes share a row: way w takes the row's non-zeros w, w + 16, ... and each of its lanes one
-// piece of the gathered row, so a wave runs 4 / L rows and a gather moves only the batch's own bytes of a source row.
-// The 16 partial sums meet in a fixed tree that does not depend on L: a board's sums have the same bits whatever the
-// batch around it.  What bounds it: the L1's line fills, one 128-byte line per gather whatever the gather uses of it
-// (10.5M non-zeros over 16-byte rows in 73 us, 143 G lines/s, where the swept kernel took 110 us: it issues 1.27
-// gathers per non-zero and finds two thirds of its 128-byte rows in the L2, this one nearly all of its 16-byte rows).
+// half or 8 float columns).  16 ways of L lanes share a row: way w takes the row's non-zeros w, w + 16, ... and each of
+// its lanes one piece of the gathered row, so a wave runs 4 / L rows and a gather moves only the batch's own bytes of a
+// source row.  The 16 partial sums meet in a fixed tree that does not depend on L: a board's sums have the same bits in
+// every batch that runs here (staged and wide steps add in other orders).  What bounds it: the L1's line fills, one
+// 128-byte line per gather whatever the gather uses of it (10.5M non-zeros over 16-byte rows in 73 us, 143 G lines/s,
+// where the swept kernel took 110 us: it issues 1.27 gathers per non-zero and finds two thirds of its 128-byte rows in
+// the L2, this one nearly all of its 16-byte rows).  A hub row stays with its 16 ways, 64 non-zeros a round.
 template <typename S, typename U, int V, int L, bool TORCH_LERP>
 __global__ __launch_bounds__(256) void k_state_step_narrow(const StepArgs<S, U> a) {
   constexpr int WAYS = 16, P = WAYS * L, RW = 64 / P, UNR = 4;
@@ -778,8 +779,8 @@ __global__ __launch_bounds__(256) void k_state_step_narrow(const StepArgs<S, U> 
 // rows' records of that band (StageTables) in order, 16 lanes per row.  It stores each row's sum over the band to
 // partials (bands, nrows, NC); k_stage_finish adds a row's bands.  What is left is the record stream from HBM: 10.5M
 // non-zeros (84 MB) of a half column in 31 us and 5 us for the finish, against 73 us in the narrow kernel and 110 in
-// the swept one.  The bands of a row block run on one XCD (workgroup b
-// on XCD b mod 8), whose L2 then reads the records' lines once.
+// the swept one.  The bands of a row block run on one XCD (workgroup b on XCD b mod 8), whose L2 then reads the records'
+// lines once.
 template <typename S, int NC>
 __global__ __launch_bounds__(1024) void k_stage_sums(const int32_t *__restrict__ start, const int2 *__restrict__ colval,
                                                      const S *__restrict__ xprev, int32_t prev_rows, int32_t nrows,

@@ -488,8 +488,8 @@ int64_t fly_profile_launches(int32_t *cls, double *ms, int64_t cap);
  * half-state elements per lane of those row slots (8 = 16 bytes, 16 = 32 bytes; 0 = automatic); "spmm_groups":
  * lane groups of fly_spmm on 16-byte lanes (2, 4, 8; 0 = automatic); "gemm_tile": workgroup tile of the dense
  * maps (1 = 64 x 64, 2 = 128 x 64, 3 = 128 x 128, or 10 TM + TN for 32 TM x 32 TN with TM in {2, 3, 4} and TN in
- * {2, 4, 5}; 0 = automatic); "gemm_splits": parts of the head's K loop, 1 to 8 (0 = automatic); "step_lds": bytes of LDS each state-step workgroup reserves, which caps the
- * workgroups a CU runs at once (0 = none); "download_blocks": workgroups of fly_evaluator_download when its call
+ * {2, 4, 5}; 0 = automatic); "gemm_splits": parts of the head's K loop, 1 to 8 (0 = automatic); "step_lds": bytes of
+ * LDS each state-step workgroup reserves, which caps the workgroups a CU runs at once (0 = none); "download_blocks": workgroups of fly_evaluator_download when its call
  * passes 0 (0 = 16); "swept": -1 keeps the long-row steps on the grouped kernel instead of the banded sweep, 1
  * sweeps every step with a matrix whatever its size (small graphs in tests), 0 = the size rule; "sweep_bands":
  * source bands of the sweep, 3 or 4 (0 = 4); "sweep_order": -1 lets the swept waves take their rows in the initial
@@ -501,8 +501,9 @@ int64_t fly_profile_launches(int32_t *cls, double *ms, int64_t cap);
  * rows in passes of 3 slots (0: 6 when a wave owns over 24 rows); "sweep_pipe": the next four rounds' gathers in
  * flight during the sums, 0 in passes of 3 slots, 1 also of 6, -1 never; "sweep_last_sync": 1 makes a swept
  * workgroup's waves also meet after a chunk's last band (0: they go on to the epilogue at once); "nt_load": 1 reads
- * the carried state with non-temporal loads; "narrow": -1 runs small batches (up to 64 bytes of state per row) on the
- * wide batches' kernels and state layout (0: on their own).  Every selectable shape computes the same function. */
+ * the carried state with non-temporal loads; "narrow": 0 gives small batches (up to 64 bytes of
+ * state per row) rows of their own bytes, and up to 32 bytes kernels of their own, -1 the wide batches' rows and
+ * kernels.  Every selectable shape computes the same function. */
 int fly_set_tuning(const char *key, int64_t value);
 /* The current default of a tuning key (as fly_set_tuning left it). */
 int fly_get_tuning(const char *key, int64_t *value);
