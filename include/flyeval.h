@@ -4,12 +4,12 @@
  * Every entry point returns an int status (FLY_OK = 0) and never throws; on failure
  * fly_last_error() returns a message for the calling thread.  Pointers named *_dev are device
  * pointers owned by the caller (torch tensors on the Python side); the library never frees them.
- * The library owns only what its create functions return (cones and plans) and frees it in the
- * matching destroy.  `stream` is a hipStream_t passed as void* (torch's current stream); every
+ * The library owns only what its create functions return (cones, plans, dense plans, sweeps) and
+ * releases it in the matching destroy (see fly_trim_memory).  `stream` is a hipStream_t passed as void* (torch's current stream); every
  * launch goes on it.  Only the create functions synchronise (they read sizes back to the host);
  * the forward entry points are asynchronous.  Index arrays are int32, the graph is CSR of
  * W[post, pre] (row = postsynaptic neuron).  A created object is immutable apart from the cone's cache of sweep
- * tables, which takes a lock: plans may be created and forwards run from several threads, each with its own
+ * tables and a sweep's tables for one or two positions, which take locks: plans may be created and forwards run from several threads, each with its own
  * workspace and stream.  fly_set_tuning changes the defaults of objects created afterwards.
  *
  * Reference interfaces replaced (paths relative to the alpha-fly repository):
@@ -44,6 +44,7 @@
  *   fly_train_step_*      chessfly/brain.py:313-327 under autograd (clamp, index_add, index_copy, lerp and their
  *                         gradients)
  *   fly_model_forward_static  no counterpart: the model forward for callers that cannot allocate
+ *   fly_trim_memory       no counterpart: the idle device memory of destroyed objects, back to the runtime
  *   fly_profile_*, fly_set_tuning, fly_get_tuning  measurement and launch-shape choices (timing scripts)
  */
 #ifndef FLYEVAL_H
