@@ -321,6 +321,23 @@ struct Vec {
     else
       *p = v[0];
   }
+  // The first n columns at p (zeros for the others), in one load where all V are there and p is aligned (`wide`).
+  static __device__ __forceinline__ Vec load_some(const float *p, int32_t n, bool wide) {
+    if (wide && n >= V) return load(p);
+    Vec r;
+#pragma unroll
+    for (int i = 0; i < V; ++i) r.v[i] = i < n ? p[i] : 0.0f;
+    return r;
+  }
+  __device__ __forceinline__ void store_some(float *p, int32_t n, bool wide) const {
+    if (wide && n >= V) {
+      store(p);
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      if (i < n) p[i] = v[i];
+  }
 };
 
 struct StepFwdArgs {
@@ -336,11 +353,15 @@ struct StepFwdArgs {
   int64_t ldh;
   float hmax;
   int32_t rows, batch, has_s;
+  int32_t u_wide;              // RAGGED: u's rows start on 16 bytes too
 };
 
 // y = s + k + u[usrc];  x = clamp(y, 0, hmax);  p = h_{t-1}[prev] or pdef;  h = lerp(p, x, a).  One wave per
-// row, V columns per lane.
-template <int V>
+// row, V columns per lane.  RAGGED: the batch is no multiple of V; the rows start on 16 bytes, u's perhaps not, and the
+// columns behind the batch are neither read nor written.  It runs from 129 positions on, where one column per lane takes
+// a third pass (full-size network, ms per forward and backward, with one column per lane and ragged: 145 positions 7.92 /
+// 7.87, 201 9.95 / 9.88; below, 67 positions 5.92 / 5.94, 127 6.88 / 6.90, 27 4.45 / 4.49).
+template <int V, bool RAGGED>
 __global__ __launch_bounds__(256) void k_train_fwd(const StepFwdArgs a) {
   const uint32_t row = blockIdx.x * 4u + (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (row >= (uint32_t)a.rows) return;
@@ -352,9 +373,10 @@ __global__ __launch_bounds__(256) void k_train_fwd(const StepFwdArgs a) {
   const float *ur = us >= 0 ? a.u + (int64_t)us * a.ldu : nullptr;
   const float *pr = pv >= 0 ? a.hprev + (int64_t)pv * a.ldp : nullptr;
   for (int32_t c = lane * V; c < a.batch; c += 64 * V) {
-    Vec<V> s = a.has_s ? Vec<V>::load(sy + c) : Vec<V>::fill(0.0f);
-    const Vec<V> u = ur ? Vec<V>::load(ur + c) : Vec<V>::fill(0.0f);
-    const Vec<V> p = pr ? Vec<V>::load(pr + c) : Vec<V>::fill(pd);
+    const int32_t n = RAGGED ? a.batch - c : V;
+    Vec<V> s = a.has_s ? Vec<V>::load_some(sy + c, n, true) : Vec<V>::fill(0.0f);
+    const Vec<V> u = ur ? Vec<V>::load_some(ur + c, n, !RAGGED || a.u_wide) : Vec<V>::fill(0.0f);
+    const Vec<V> p = pr ? Vec<V>::load_some(pr + c, n, true) : Vec<V>::fill(pd);
     Vec<V> out;
 #pragma unroll
     for (int i = 0; i < V; ++i) {
@@ -362,8 +384,8 @@ __global__ __launch_bounds__(256) void k_train_fwd(const StepFwdArgs a) {
       s.v[i] = y;
       out.v[i] = lerp_torch(p.v[i], fminf(fmaxf(y, 0.0f), a.hmax), al);
     }
-    s.store(sy + c);
-    out.store(h + c);
+    s.store_some(sy + c, n, true);
+    out.store_some(h + c, n, true);
   }
 }
 
@@ -385,6 +407,7 @@ struct StepBwdArgs {
   int64_t ldgh;
   float hmax;
   int32_t rows, batch;
+  int32_t gu_wide;             // RAGGED: gu's rows start on 16 bytes too
 };
 
 __device__ __forceinline__ float wave_sum(float v) {
@@ -395,8 +418,8 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 // The gradients of h = lerp(p, clamp(y, 0, hmax), a): dL/dy = g a [0 <= y <= hmax] (torch.clamp passes the
 // bounds), dL/dp = g (1 - a), dL/da = sum_b g (x - p); dL/dk = sum_b dL/dy; dL/dpdef = sum_b dL/dp on rows
-// that are not carried; carried rows pass dL/dp to h_{t-1}[prev]; input rows add dL/dy to u[usrc].
-template <int V>
+// that are not carried; carried rows pass dL/dp to h_{t-1}[prev]; input rows add dL/dy to u[usrc].  RAGGED as above.
+template <int V, bool RAGGED>
 __global__ __launch_bounds__(256) void k_train_bwd(const StepBwdArgs a) {
   const uint32_t row = blockIdx.x * 4u + (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (row >= (uint32_t)a.rows) return;
@@ -411,11 +434,13 @@ __global__ __launch_bounds__(256) void k_train_bwd(const StepBwdArgs a) {
   float *gur = us >= 0 ? a.gu + (int64_t)us * a.ldgu : nullptr;
   float sk = 0.0f, sa = 0.0f, sp = 0.0f;
   for (int32_t c = lane * V; c < a.batch; c += 64 * V) {
-    const Vec<V> g = Vec<V>::load(gr + c), y = Vec<V>::load(yr + c);
-    const Vec<V> p = pr ? Vec<V>::load(pr + c) : Vec<V>::fill(pd);
+    const int32_t n = RAGGED ? a.batch - c : V;
+    const Vec<V> g = Vec<V>::load_some(gr + c, n, true), y = Vec<V>::load_some(yr + c, n, true);
+    const Vec<V> p = pr ? Vec<V>::load_some(pr + c, n, true) : Vec<V>::fill(pd);
     Vec<V> gy, gp;
 #pragma unroll
     for (int i = 0; i < V; ++i) {
+      if (RAGGED && i >= n) break;   // a column behind the batch adds nothing, whatever p is
       const float x = fminf(fmaxf(y.v[i], 0.0f), a.hmax);
       gy.v[i] = (y.v[i] >= 0.0f && y.v[i] <= a.hmax) ? g.v[i] * al : 0.0f;
       gp.v[i] = g.v[i] * (1.0f - al);
@@ -423,13 +448,14 @@ __global__ __launch_bounds__(256) void k_train_bwd(const StepBwdArgs a) {
       sa += g.v[i] * (x - p.v[i]);
       sp += gp.v[i];
     }
-    gy.store(gyr + c);
-    if (ghr) gp.store(ghr + c);
+    gy.store_some(gyr + c, n, true);
+    if (ghr) gp.store_some(ghr + c, n, true);
     if (gur) {
-      Vec<V> u = Vec<V>::load(gur + c);
+      const bool wide = !RAGGED || a.gu_wide;
+      Vec<V> u = Vec<V>::load_some(gur + c, n, wide);
 #pragma unroll
       for (int i = 0; i < V; ++i) u.v[i] += gy.v[i];
-      u.store(gur + c);
+      u.store_some(gur + c, n, wide);
     }
   }
   sk = wave_sum(sk);
@@ -1338,14 +1364,15 @@ extern "C" int fly_train_step_forward(int64_t rows, int64_t batch, float *s_y, i
     FLY_REQUIRE(!prev || (hprev && ldp >= batch), "carried rows need the previous state");
     LaunchTimer timer(FLY_K_OTHER, as_stream(stream));
     StepFwdArgs a{s_y, lds, k, pdef, alpha, prev, usrc, u, ldu, hprev, ldp, h, ldh, h_max, (int32_t)rows,
-                  (int32_t)batch, has_s != 0};
-    const bool v4 = batch % 4 == 0 && vec4_ok(s_y, lds) && vec4_ok(h, ldh) && (!usrc || vec4_ok(u, ldu)) &&
-                    (!prev || vec4_ok(hprev, ldp));
+                  (int32_t)batch, has_s != 0, usrc && vec4_ok(u, ldu)};
+    const bool rows_ok = vec4_ok(s_y, lds) && vec4_ok(h, ldh) && (!prev || vec4_ok(hprev, ldp));
     const dim3 grid(blocks_for(rows, 4)), block(256);
-    if (v4)
-      hipLaunchKernelGGL(k_train_fwd<4>, grid, block, 0, as_stream(stream), a);
+    if (batch % 4 == 0 && rows_ok && (!usrc || a.u_wide))
+      hipLaunchKernelGGL((k_train_fwd<4, false>), grid, block, 0, as_stream(stream), a);
+    else if (batch > 128 && rows_ok)
+      hipLaunchKernelGGL((k_train_fwd<4, true>), grid, block, 0, as_stream(stream), a);
     else
-      hipLaunchKernelGGL(k_train_fwd<1>, grid, block, 0, as_stream(stream), a);
+      hipLaunchKernelGGL((k_train_fwd<1, false>), grid, block, 0, as_stream(stream), a);
     check_launch("train step forward");
   });
 }
@@ -1364,14 +1391,16 @@ extern "C" int fly_train_step_backward(int64_t rows, int64_t batch, const float 
     FLY_REQUIRE(!prev || (hprev && ghprev && ldp >= batch && ldgh >= batch), "carried rows need the previous state");
     LaunchTimer timer(FLY_K_OTHER, as_stream(stream));
     StepBwdArgs a{g, ldg, y, ldy, pdef, alpha, prev, usrc, hprev, ldp, gy, ldgy, gk, ga, gpdef, gu, ldgu, ghprev,
-                  ldgh, h_max, (int32_t)rows, (int32_t)batch};
-    const bool v4 = batch % 4 == 0 && vec4_ok(g, ldg) && vec4_ok(y, ldy) && vec4_ok(gy, ldgy) &&
-                    (!usrc || vec4_ok(gu, ldgu)) && (!prev || (vec4_ok(hprev, ldp) && vec4_ok(ghprev, ldgh)));
+                  ldgh, h_max, (int32_t)rows, (int32_t)batch, usrc && vec4_ok(gu, ldgu)};
+    const bool rows_ok = vec4_ok(g, ldg) && vec4_ok(y, ldy) && vec4_ok(gy, ldgy) &&
+                         (!prev || (vec4_ok(hprev, ldp) && vec4_ok(ghprev, ldgh)));
     const dim3 grid(blocks_for(rows, 4)), block(256);
-    if (v4)
-      hipLaunchKernelGGL(k_train_bwd<4>, grid, block, 0, as_stream(stream), a);
+    if (batch % 4 == 0 && rows_ok && (!usrc || a.gu_wide))
+      hipLaunchKernelGGL((k_train_bwd<4, false>), grid, block, 0, as_stream(stream), a);
+    else if (batch > 128 && rows_ok)
+      hipLaunchKernelGGL((k_train_bwd<4, true>), grid, block, 0, as_stream(stream), a);
     else
-      hipLaunchKernelGGL(k_train_bwd<1>, grid, block, 0, as_stream(stream), a);
+      hipLaunchKernelGGL((k_train_bwd<1, false>), grid, block, 0, as_stream(stream), a);
     check_launch("train step backward");
   });
 }

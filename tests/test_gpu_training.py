@@ -710,7 +710,7 @@ def test_full_scale_train_step_gradients_match_the_oracle(full_net, batch):
         _close(got[name], want[name], 1e-3, name)
 
 
-@pytest.mark.parametrize("batch", [1, 3, 25, 36, 66, 201])
+@pytest.mark.parametrize("batch", [1, 3, 25, 36, 66, 129, 201])
 @pytest.mark.parametrize("swept", [False, True])
 def test_cone_gradients_of_ragged_batches_match_the_oracle(batch, swept):
     """forward_io under autograd at batches that are no multiple of 4 or of 32, which run with columns of zeros behind them:
